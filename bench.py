@@ -352,7 +352,7 @@ def exact_decode(path, ids, warmup, steps):
     """The token-identical path: the same Llama-3-8B-shaped file opened in
     exact mode (every kernel in the reference CPU engine's float order, so
     each step's logits equal its sml_forward bit for bit), the same prompt
-    read exactly (batched: 64-position chunks through the reference-order
+    read exactly (batched: 512-position chunks through the reference-order
     GEMM and attention, equal to stepping it bit for bit), then `warmup`
     untimed and `steps` timed greedy tokens at the fast line's positions."""
     dec = sa.Decoder(path, n_ctx=N_CTX, exact=True)

@@ -40,10 +40,10 @@ const float * sml_gpu_step(int tok, int pos);
 int sml_gpu_layers(int * of);
 
 // How a prompt is read: 0 a token at a time through the decode graph; 1 (the
-// default) batched in chunks of 32 positions (16 with MoE layers) with every
+// default) batched in chunks of 512 positions (16 with MoE layers) with every
 // product in the GEMV's arithmetic, equal to stepping bit for bit; 2 batched
 // with the Q4 products on the matrix cores (MFMA), equal to float rounding.
-// Exact mode (SML_EXACT=1) takes 2 as 1: chunks of 64 positions in the
+// Exact mode (SML_EXACT=1) takes 2 as 1: chunks of 512 positions in the
 // reference CPU path's float order, equal to its stepping bit for bit.
 // replaces sml/sml-gpu.h:26 (sml/sml-gpu-fwd.c:2420-2423)
 void sml_gpu_prompt_mode(int level);

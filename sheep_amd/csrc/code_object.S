@@ -1,5 +1,5 @@
-// The gfx950 code objects built from kernels.hip and ingest.hip, linked into
-// the library as read-only data and loaded with hipModuleLoadData at init.
+// The gfx950 code objects built from kernels.hip, ingest.hip and prompt.hip,
+// linked into the library as read-only data and loaded with hipModuleLoadData at init.
     .section .rodata
     .balign 4096
     .global sml_code_object
@@ -16,5 +16,13 @@ sml_ingest_object:
     .incbin "ingest.hsaco"
     .global sml_ingest_object_end
 sml_ingest_object_end:
+    .byte 0
+    .balign 4096
+    .global sml_prompt_object
+    .type sml_prompt_object, @object
+sml_prompt_object:
+    .incbin "prompt.hsaco"
+    .global sml_prompt_object_end
+sml_prompt_object_end:
     .byte 0
     .section .note.GNU-stack,"",@progbits

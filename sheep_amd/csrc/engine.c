@@ -97,11 +97,10 @@ static struct {
     uint16_t ** kc_tab, ** vc_tab;   // device tables of every slot's cache base
     float * mpart;             // attention partials of every sequence of a batch
     size_t mpart_floats;
-    int xchunk;                // exact mode's prompt chunk: its rows' scores fit in mpart
     int32_t * iota;            // device [n_ctx]: 0, 1, 2, ... (prompt chunk positions)
     int32_t * slotid;          // device [MAX_SLOTS][rrows]: row s filled with s
     int rrows;                 // rows of the batched body's buffers: max(MAX_SLOTS, pb)
-    int pb;                    // positions per chunk of a level-2 prompt
+    int pb;                    // positions per chunk of a batched prompt
     int rows_ok;               // 1: the batched body can run this model (-1: not checked yet)
     int rows_ready;            // the batched body's buffers are allocated
     // A layer split: layers below nres keep their matrices in HBM. The rest
@@ -708,7 +707,7 @@ static void setup(const char * path, int want_ctx, int gpu_layers) {
     // open does (sml/sml-gpu-fwd.c:2371-2375); in exact mode level 1 is the
     // reference-order batched prompt where every product takes it (rows_check)
     G.prompt_level = env_int("SML_GPU_PP", 1) == 0 ? 0 : 1;
-    // level-2 chunk: SML_PB positions (16..4096, default 512); MoE layers
+    // prompt chunk: SML_PB positions (16..4096, default 512); MoE layers
     // take at most MAX_SLOTS rows per call
     G.pb = env_int("SML_PB", 512);
     if (G.pb < MAX_SLOTS) G.pb = MAX_SLOTS;
@@ -945,11 +944,6 @@ static void rows_alloc(void) {
     if (part_pb > part) part = part_pb;
     G.mpart = dalloc(part * 4);
     G.mpart_floats = part;
-    // exact mode reads a prompt in chunks whose reference-order scores
-    // ([rows][H][n_ctx] floats) fit in the partials buffer: at most 64 rows
-    G.xchunk = (int) (part / ((size_t) G.H * (size_t) G.n_ctx));
-    if (G.xchunk > 64) G.xchunk = 64;
-    if (G.xchunk > G.rrows) G.xchunk = G.rrows;
     hx_kpart();                                     // the split-K products' buffer, before any capture
     G.kc_tab = dalloc(S * sizeof(void *));
     G.vc_tab = dalloc(S * sizeof(void *));
@@ -1019,18 +1013,31 @@ static void rows_layer(int L, int ns, const int32_t * pos, const int32_t * slot,
     // that to its own launch)
     const int fuse_q = y->perm_o < 0 &&
                        (!sb || (!causal && G.H % 2 == 0 && G.hd == 128 && env_int("SML_MERGE_Q256", 1)));
-    if (regime == GEMM_REF) {
-        // exact mode: one sequence (slot 0), the reference's order
-        if (!causal) hx_failf("exact mode batches prompts only");
-        op_attention_rows_exact(G.st, G.mqkv, (int) qkv, G.kc + (size_t) L * G.n_ctx * kvd,
-                                G.vc + (size_t) L * G.n_ctx * kvd, G.rc, G.rs, pos, ns, G.H, G.KV, G.n_ctx,
-                                G.pos_cap, G.mpart, G.matt, fuse_q ? G.maq : NULL, fuse_q ? G.mas : NULL,
-                                fuse_q ? G.masum : NULL);
-    } else {
-        op_attention_batch(G.st, G.mqkv, (int) qkv, G.kc_tab, G.vc_tab, slot, (size_t) L * G.n_ctx * kvd,
-                           G.rc, G.rs, pos, ns, G.H, G.KV, G.hd, G.n_ctx, G.pos_cap, G.mpart, G.matt,
-                           fuse_q ? G.maq : NULL, fuse_q ? G.mas : NULL, fuse_q ? G.masum : NULL,
-                           causal ? (regime == GEMM_EXACT ? 1 : 2) : 0, gemm_exact(regime, ns), sb);
+    // a level-1 or exact-mode prompt chunk attends in slices of rows whose
+    // partials (scores) fit the buffer; a slice's rows see the cache rows that
+    // it and the slices before it wrote
+    int sl = ns;
+    if (regime == GEMM_REF) sl = (int) (G.mpart_floats / ((size_t) G.H * (size_t) G.n_ctx));
+    else if (causal && regime == GEMM_EXACT) sl = op_attention_rows(G.H, G.KV, G.hd, G.n_ctx, G.pos_cap, G.mpart_floats);
+    if (sl < 1) hx_failf("attention partials of no row");
+    for (int r0 = 0; r0 < ns; r0 += sl) {
+        const int nr = ns - r0 < sl ? ns - r0 : sl;
+        const size_t ro = (size_t) r0 * hq;
+        int8_t * aq = fuse_q ? G.maq + ro : NULL;
+        float * as = fuse_q ? G.mas + ro / 32 : NULL;
+        int32_t * au = fuse_q ? G.masum + ro / 32 : NULL;
+        if (regime == GEMM_REF) {
+            // exact mode: one sequence (slot 0), the reference's order
+            if (!causal) hx_failf("exact mode batches prompts only");
+            op_attention_rows_exact(G.st, G.mqkv + (size_t) r0 * qkv, (int) qkv, G.kc + (size_t) L * G.n_ctx * kvd,
+                                    G.vc + (size_t) L * G.n_ctx * kvd, G.rc, G.rs, pos + r0, nr, G.H, G.KV, G.n_ctx,
+                                    G.pos_cap, G.mpart, G.matt + ro, aq, as, au);
+        } else {
+            op_attention_batch(G.st, G.mqkv + (size_t) r0 * qkv, (int) qkv, G.kc_tab, G.vc_tab, slot + r0,
+                               (size_t) L * G.n_ctx * kvd, G.rc, G.rs, pos + r0, nr, G.H, G.KV, G.hd, G.n_ctx,
+                               G.pos_cap, G.mpart, G.matt + ro, aq, as, au,
+                               causal ? (regime == GEMM_EXACT ? 1 : 2) : 0, gemm_exact(regime, ns), sb);
+        }
     }
     if (!fuse_q) {
         pp[0] = pdev(y->perm_o);
@@ -1098,11 +1105,11 @@ static void launch_rows(int ns, const int32_t * tok, const int32_t * pos, const 
 // matrix streamed once per chunk; the last position's residual then goes
 // through the decode tail (final norm, head, greedy pick). The ids are
 // already in G.hist.
-//  - level 1: chunks of 32 positions (16 with MoE layers); every product is
-//    the GEMV's arithmetic and the attention the decode kernel's, so the
+//  - level 1: chunks of pb (512) positions (16 with MoE layers); every product
+//    is the GEMV's arithmetic and the attention the decode kernel's, so the
 //    cache, the residuals and the logits equal reading the prompt a token at
 //    a time, bit for bit.
-//  - exact mode: chunks of 64 through the reference-order GEMM and attention.
+//  - exact mode: chunks of pb through the reference-order GEMM and attention.
 //  - level 2: chunks of pb (512) positions in the reference's prompt regime
 //    (activations per 256 values, integer superblock sums: the CPU engine's
 //    default prompt arithmetic, sml/sml-run.c:1929-1945), Q4 products on the
@@ -1150,16 +1157,11 @@ static void prefill_layers(int slot, int pos0, int n, int chunk, int regime) {
 static void prefill_rows(int slot, int pos0, int n) {
     if (slot != 0 && mid_on()) hx_failf("a middle stage serves slot 0 only");
     rows_alloc();
-    // exact mode: the reference-order products and attention, in chunks of
-    // xchunk positions
     const int regime = G.exact ? GEMM_REF : G.prompt_level >= 2 ? GEMM_PER256 : GEMM_EXACT;
-    // level 1: 32 positions a chunk (the exact-regime GEMM's widest form),
-    // 16 where MoE layers take part (the expert kernels' row limit)
-    int moe = 0;
-    for (int L = 0; L < G.n_layer; L++) moe |= G.L[L].moe != NULL;
-    const int c1 = moe ? MAX_SLOTS : (G.rrows < 32 ? G.rrows : 32);
-    const int chunk = G.exact ? G.xchunk : G.prompt_level >= 2 ? G.pb : c1;
-    if (chunk < 1) hx_failf("exact prompt chunk of %d rows", chunk);
+    // every regime reads pb positions a chunk (each weight matrix streams
+    // once per chunk), MAX_SLOTS where MoE layers take part (the expert
+    // kernels' row limit: pb is MAX_SLOTS then)
+    const int chunk = G.pb;
     if (G.nres < G.n_layer) {
         prefill_layers(slot, pos0, n, chunk, regime);
         return;

@@ -20,6 +20,7 @@ typedef struct {
     int       device;
     hipModule_t mod;
     hipModule_t mod_ingest;       // the ingest kernels (built without contraction)
+    hipModule_t mod_prompt;       // the prompt-reading kernels (sml_pp_*)
     int       ncu;                // compute units of the device
     long      fail_after;         // test hook: fail the Nth HIP call from now (< 0: off)
     long      calls;              // HIP calls made through HX() so far

@@ -12,24 +12,7 @@
 // the reference's per-group float epilogue (sml/sml-kernel.c:2054-2063):
 // step*(s*dot) + min*(s*sum).
 #include <hip/hip_runtime.h>
-#include "kargs.h"
-
-#define WAVE 64
-
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef unsigned int v4u __attribute__((ext_vector_type(4)));
-typedef unsigned int v2u __attribute__((ext_vector_type(2)));
-
-// Global-memory views of device pointers. A pointer read from a table in
-// device memory (expert matrices, KV slots) or selected at run time is
-// generic to the compiler, and loads through it become flat loads. A flat
-// load counts against the LDS/scalar wait counter as well as the vector
-// one, so every LDS or scalar-load wait after it also waits for it, and the
-// vector waits can no longer be partial: a kernel that overlaps its weight
-// or KV stream with LDS work then runs serially. Every such pointer here
-// points to global memory.
-#define GLOBAL __attribute__((address_space(1)))
-template <typename T> __device__ __forceinline__ T gld(const void * p) { return *(const GLOBAL T *) p; }
+#include "dev.h"
 
 // The greedy pick's order: the larger value, the lower index on a tie; NaN is
 // never taken (the reference's loop, sml/sml-run.c:3539-3544).
@@ -42,9 +25,6 @@ __device__ __forceinline__ void amax_take(float v, int i, float & bv, int & bi) 
 // comes before loads the source issues earlier (the GEMV's weights).
 __device__ __forceinline__ void pin(float & v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ void pin(int & v) { asm volatile("" : "+v"(v)); }
-
-__device__ __forceinline__ float h2f(uint16_t h) { return (float) __builtin_bit_cast(_Float16, h); }
-__device__ __forceinline__ uint16_t f2h(float f) { return __builtin_bit_cast(uint16_t, (_Float16) f); }
 
 __device__ __forceinline__ float wave_sum(float v) {
     #pragma unroll
@@ -102,59 +82,6 @@ __device__ __forceinline__ float max32(float v) { v = max16(v); return fmaxf(v, 
 __device__ __forceinline__ int isum32(int v) { v = isum16(v); return v + __builtin_amdgcn_ds_swizzle(v, 0x401F); }
 
 __device__ __forceinline__ int dot4(unsigned a, int b, int c) { return __builtin_amdgcn_sdot4((int) a, b, c, false); }
-
-// 4 bits (one per column) -> 4 bytes of 0/1
-__device__ __forceinline__ unsigned bits4_to_bytes(unsigned nib) { return (nib * 0x00204081u) & 0x01010101u; }
-
-// ---------------------------------------------------------------- chunks
-//
-// A chunk is 16 bytes of a row's nibble plane: columns 16*(c&1)..+15 of the
-// group pair (c&~1, c|1) -- byte i's low nibble belongs to the first group,
-// its high nibble to the second (the FLAT layout, sml/sml-kernel.c:2140-2156).
-// Lane c of a row loads chunk c, so 64 lanes read 1 KB of contiguous bytes
-// per instruction; the other planes' bytes for the same weights are equally
-// contiguous across lanes (a 2-bit pack serves two lanes, a 1-bit word pair
-// serves a lane pair). Plane orders per width follow
-// tooling/sml_quantize.py:104-106: Q2 [2], Q3 [2,1], Q4 [4], Q5 [4,1],
-// Q6 [2,4] (the 2-bit plane holds bits 4-5), Q7 [4,2,1], Q8 [4,4].
-template <int NB> struct Planes {
-    static constexpr bool N4 = NB == 4 || NB == 5 || NB == 6 || NB == 7 || NB == 8;
-    static constexpr bool N2 = NB == 2 || NB == 3 || NB == 6 || NB == 7;
-    static constexpr bool N1 = NB == 3 || NB == 5 || NB == 7;
-    static constexpr int P4 = NB == 6 ? 1 : 0;
-    static constexpr int P2 = NB == 7 ? 1 : 0;
-    static constexpr int P1 = NB == 7 ? 2 : 1;
-    // bytes of each plane per row for `cols` weights
-    static __device__ __forceinline__ size_t b4(int cols) { return (size_t) cols / 2; }
-    static __device__ __forceinline__ size_t b2(int cols) { return (size_t) cols / 4; }
-    static __device__ __forceinline__ size_t b1(int cols) { return (size_t) cols / 8; }
-};
-
-template <bool NT, typename T>
-__device__ __forceinline__ T ld(const T * p) {
-    const GLOBAL T * g = (const GLOBAL T *) p;
-    if constexpr (NT) return __builtin_nontemporal_load(g);
-    else return *g;
-}
-
-template <int NB> struct ChunkW {
-    v4u n4;                       // nibble plane word (or zeros)
-    v4u h4;                       // Q8 high nibbles
-    v4u t2;                       // 2-bit pack half
-    v2u o1;                       // 1-bit words of the group pair
-};
-
-// Chunk c of one row: pl[] are the planes' bases (uniform), ro[] the row's
-// byte offset in each plane. Offsets are 32-bit so the loads address as
-// uniform base + per-lane offset, which keeps one VGPR per address.
-template <int NB, bool NT>
-__device__ __forceinline__ void load_chunk(ChunkW<NB> & w, const uint8_t * const * pl, const uint32_t * ro, int c) {
-    using P = Planes<NB>;
-    if constexpr (P::N4) w.n4 = ld<NT>((const v4u *) (pl[P::P4] + (ro[P::P4] + (uint32_t) c * 16u)));
-    if constexpr (NB == 8) w.h4 = ld<NT>((const v4u *) (pl[1] + (ro[1] + (uint32_t) c * 16u)));
-    if constexpr (P::N2) w.t2 = ld<NT>((const v4u *) (pl[P::P2] + (ro[P::P2] + (uint32_t) (c >> 2) * 32u + (uint32_t) (c & 1) * 16u)));
-    if constexpr (P::N1) w.o1 = ld<NT>((const v2u *) (pl[P::P1] + (ro[P::P1] + (uint32_t) (c >> 1) * 8u)));
-}
 
 // partial dots of chunk c over its 16 columns: da for group c&~1 against
 // xa, db for group c|1 against xb
@@ -233,27 +160,6 @@ __device__ __forceinline__ int quant1(float v, float is) {
     const float r = __builtin_rintf(v * is);
     int t = (r >= -2147483648.0f && r < 2147483648.0f) ? (int) r : (int) 0x80000000u;
     return t > 127 ? 127 : t < -127 ? -127 : t;
-}
-
-// SiLU as the reference's x86 build computes it (sml_exp_ps + silu_mul,
-// sml/sml-run.c:393-426): the argument clamped to [-88, 88], f = x*log2(e),
-// r = f rounded half-even, 2^(f-r) by a degree-5 Horner chain of FMAs, and
-// 1 + p*2^r folded into one FMA (how that build's compiler contracts it);
-// then g / d. Contraction is off so f and f - r round as written.
-__device__ __forceinline__ float silu_ref(float g) {
-    #pragma clang fp contract(off)
-    float x = 0.0f - g;
-    x = fminf(fmaxf(x, -88.0f), 88.0f);
-    const float f = x * 1.44269504088896341f;
-    const float r = __builtin_rintf(f);
-    const float t = f - r;
-    float p = __builtin_fmaf(1.3697664e-3f, t, 8.3013611e-3f);
-    p = __builtin_fmaf(p, t, 5.5826318e-2f);
-    p = __builtin_fmaf(p, t, 2.4022652e-1f);
-    p = __builtin_fmaf(p, t, 6.9314718e-1f);
-    p = __builtin_fmaf(p, t, 1.0f);
-    const float sc = __builtin_bit_cast(float, ((int) r + 127) << 23);
-    return g / __builtin_fmaf(p, sc, 1.0f);
 }
 
 // expf of the C library the reference runs on (glibc 2.35 on x86-64 with FMA),
@@ -4286,171 +4192,6 @@ extern "C" __global__ __launch_bounds__(256) void sml_gemm_ksum(const sml_kksum 
     if (a.resid) v = a.resid[i] + v;
     a.y[i] = v;
 }
-
-
-
-// ---------------------------------------------------------------- batched GEMM in the reference's order (exact mode)
-//
-// Y[p][r] = W.a[p] for the positions p of an exact-mode prompt chunk, each
-// output the exact GEMV's (gemv_body EX, the reference's flat4 kernel,
-// sml/sml-kernel.c:572-727) bit for bit, the weights read once for 64
-// positions. Per-32 activations (s_g, sum_g per group). For each (row,
-// position) the reference keeps 8 float chains, chain j taking groups j,
-// j+8, ... of the row in order:
-//     v_j = fma(sd*sq_g, s_g*dot_g, v_j);  v_j = fma(md*(mq_g-127), s_g*sum_g, v_j)
-// then ((v0+v4)+(v1+v5)) + ((v2+v6)+(v3+v7)); y = resid + (v + bias).
-// The integer dot_g comes from one v_mfma_i32_16x16x32_i8 per group and
-// 16 x 16 tile (the operand layout of mgemm_q4_body: lane l holds weight row
-// l%16 and positions 4(l/16)..+3 of the wave's 16). A lane runs the chains
-// of its own (row, position) pairs over the groups in order, 8 chains x 4
-// positions in registers (x 2 for SwiGLU: gate and up), so no value crosses
-// lanes before the fold. Workgroup: 4 waves = 64 positions x 16 weight rows;
-// the waves read the same weight bytes (L1). Inputs a multiple of 256 wide
-// (no trailing half superblock: the caller checks). Q8 (NB 8: two nibble
-// planes, code = lo + 16 hi, the reference's flat8 reads the same planes
-// with the 4-bit kernel, sml/sml-kernel.c:1066-1073): dot_g = dot_lo +
-// 16 dot_hi from two MFMAs, the same integer.
-template <bool SW, int NB = 4>
-__device__ void xgemm_q4_body(const sml_kgemm & a) {
-    #pragma clang fp contract(off)
-    static_assert(NB == 4 || NB == 8, "Q4 or Q8");
-    constexpr int NP = NB == 8 ? 2 : 1;                       // nibble planes
-    typedef long v1l;
-    constexpr int NM = SW ? 2 : 1;
-    const int n = a.cols, ng = n / 32, nsb = ng / 8, rows = a.rows, m_all = a.m_all;
-    const int tid = threadIdx.x, lane = tid & 63, c = lane >> 4, i16 = lane & 15;
-    const int wave = tid >> 6;
-    const int r0 = (int) blockIdx.x * 16, p0 = (int) blockIdx.y * 64 + wave * 16;
-    const int row = min(r0 + i16, rows - 1);
-    const uint8_t * plane[NM][NP];
-    const uint8_t * fqb[NM];
-    const uint8_t * fdb[NM];
-    #pragma unroll
-    for (int k = 0; k < NM; k++) {
-        const sml_kmat & mk = a.inl ? a.m0[k] : a.mats[k];
-        #pragma unroll
-        for (int pl = 0; pl < NP; pl++) plane[k][pl] = mk.plane[pl] + (size_t) row * (n / 2) + 16 * c;
-        fqb[k] = mk.sqmq + (size_t) row * ng * 2;
-        fdb[k] = (const uint8_t *) mk.sdmd + (size_t) row * nsb * 4;
-    }
-    // the A operand's activation row (position p0 + i16) and the lane's four
-    // output positions' fields
-    const int8_t * qrow = a.q + (size_t) min(p0 + i16, m_all - 1) * n + 16 * c;
-    const float * srow[4];
-    const int32_t * urow[4];
-    #pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const size_t pr = (size_t) min(p0 + 4 * c + r, m_all - 1);
-        srow[r] = a.scale + pr * ng;
-        urow[r] = a.sums + pr * ng;
-    }
-    float ch[NM][4][8];
-    #pragma unroll
-    for (int k = 0; k < NM; k++)
-        #pragma unroll
-        for (int r = 0; r < 4; r++)
-            #pragma unroll
-            for (int j = 0; j < 8; j++) ch[k][r][j] = 0.0f;
-    for (int b = 0; b < nsb; b++) {
-        v4u w[NM][NP][2], fq[NM];
-        uint32_t fd[NM];
-        v4u aq[4];
-        #pragma unroll
-        for (int k = 0; k < NM; k++) {
-            #pragma unroll
-            for (int pl = 0; pl < NP; pl++)
-                #pragma unroll
-                for (int p = 0; p < 2; p++) w[k][pl][p] = gld<v4u>(plane[k][pl] + (size_t) b * 128 + p * 64);
-            fq[k] = gld<v4u>(fqb[k] + (size_t) b * 16);
-            fd[k] = gld<uint32_t>(fdb[k] + (size_t) b * 4);
-        }
-        #pragma unroll
-        for (int u = 0; u < 4; u++) aq[u] = *(const v4u *) (qrow + (size_t) b * 256 + u * 64);
-        float sv[4][8];
-        int uv[4][8];
-        #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const float4 s0 = *(const float4 *) (srow[r] + 8 * b), s1 = *(const float4 *) (srow[r] + 8 * b + 4);
-            const int4 u0 = *(const int4 *) (urow[r] + 8 * b), u1 = *(const int4 *) (urow[r] + 8 * b + 4);
-            sv[r][0] = s0.x; sv[r][1] = s0.y; sv[r][2] = s0.z; sv[r][3] = s0.w;
-            sv[r][4] = s1.x; sv[r][5] = s1.y; sv[r][6] = s1.z; sv[r][7] = s1.w;
-            uv[r][0] = u0.x; uv[r][1] = u0.y; uv[r][2] = u0.z; uv[r][3] = u0.w;
-            uv[r][4] = u1.x; uv[r][5] = u1.y; uv[r][6] = u1.z; uv[r][7] = u1.w;
-        }
-        // the operands: an 8-byte k-slice of every group in every lane, the
-        // same permutation of k for A and B (see mgemm_q4_body)
-        v1l av[8];
-        #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            v2u x, y;
-            xslice(aq[u], x, y);
-            av[2 * u] = (v1l) (((unsigned long) x.y << 32) | x.x);
-            av[2 * u + 1] = (v1l) (((unsigned long) y.y << 32) | y.x);
-        }
-        v2u wx[NM][NP][2], wy[NM][NP][2];
-        #pragma unroll
-        for (int k = 0; k < NM; k++)
-            #pragma unroll
-            for (int pl = 0; pl < NP; pl++)
-                #pragma unroll
-                for (int p = 0; p < 2; p++) xslice(w[k][pl][p], wx[k][pl][p], wy[k][pl][p]);
-        #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            #pragma unroll
-            for (int k = 0; k < NM; k++) {
-                v4i d = {0, 0, 0, 0};
-                #pragma unroll
-                for (int pl = NP - 1; pl >= 0; pl--) {
-                    const v2u ww = (j & 2) ? wy[k][pl][j >> 2] : wx[k][pl][j >> 2];
-                    const v2u cd = (j & 1) ? ((ww >> 4u) & 0x0F0F0F0Fu) : (ww & 0x0F0F0F0Fu);
-                    if (pl == 1) {
-                        // the high nibbles' dot, times 16, then the low ones added on
-                        d = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[j], (v1l) (((unsigned long) cd.y << 32) | cd.x), d, 0, 0, 0);
-                        #pragma unroll
-                        for (int r = 0; r < 4; r++) d[r] *= 16;
-                    } else {
-                        d = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[j], (v1l) (((unsigned long) cd.y << 32) | cd.x), d, 0, 0, 0);
-                    }
-                }
-                const uint32_t f = fq[k][j >> 1] >> (16 * (j & 1));
-                const float wsc = h2f((uint16_t) (fd[k] & 0xFFFFu)) * (float) (f & 0xFFu);
-                const float wmn = h2f((uint16_t) (fd[k] >> 16)) * ((float) ((f >> 8) & 0xFFu) - 127.0f);
-                #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const float s = sv[r][j];
-                    ch[k][r][j] = __builtin_fmaf(wsc, s * (float) d[r], ch[k][r][j]);
-                    ch[k][r][j] = __builtin_fmaf(wmn, s * (float) uv[r][j], ch[k][r][j]);
-                }
-            }
-        }
-    }
-    if (r0 + i16 >= rows) return;
-    #pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int p = p0 + 4 * c + r;
-        if (p >= m_all) continue;
-        float v[NM];
-        #pragma unroll
-        for (int k = 0; k < NM; k++) {
-            const float (&q)[8] = ch[k][r];
-            v[k] = ((q[0] + q[4]) + (q[1] + q[5])) + ((q[2] + q[6]) + (q[3] + q[7]));
-        }
-        float * y = a.y + (size_t) p * rows;
-        const int rr = r0 + i16;
-        if constexpr (SW) {
-            y[rr] = silu_ref(v[0]) * v[1];                                       // sml/sml-run.c:416-426
-        } else {
-            float o = v[0];
-            if (a.bias) o += a.bias[rr];
-            if (a.resid) o = a.resid[(size_t) p * rows + rr] + o;
-            y[rr] = o;
-        }
-    }
-}
-extern "C" __global__ __launch_bounds__(256) void sml_xgemm_q4(const sml_kgemm a) { xgemm_q4_body<false>(a); }
-extern "C" __global__ __launch_bounds__(256) void sml_xgemm_q4_s(const sml_kgemm a) { xgemm_q4_body<true>(a); }
-extern "C" __global__ __launch_bounds__(256) void sml_xgemm_q8(const sml_kgemm a) { xgemm_q4_body<false, 8>(a); }
-extern "C" __global__ __launch_bounds__(256) void sml_xgemm_q8_s(const sml_kgemm a) { xgemm_q4_body<true, 8>(a); }
 
 // ---------------------------------------------------------------- prompt GEMM on MFMA (Q4, per-256 activations)
 //

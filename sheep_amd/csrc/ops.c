@@ -1088,6 +1088,12 @@ void op_attention_rows_exact(hipStream_t st, const float * qkv, int qkv_stride, 
     hx_launch3("sml_attnx_pv", (unsigned) n_head, (unsigned) nrows, 1, 512, lds, st, &x);
 }
 
+int op_attention_rows(int n_head, int n_kv, int hd, int n_ctx, int n_pos, size_t part) {
+    const int ch = attn_split(n_kv, n_ctx, hd);
+    const size_t r = part / ((size_t) n_head * (size_t) ((n_pos + ch - 1) / ch) * (size_t) (hd + 2));
+    return r > 65535 ? 65535 : (int) r;
+}
+
 int sml_hip_attention(float * q, const float * k, const float * v, uint16_t * kcache, uint16_t * vcache,
                       const float * cos_t, const float * sin_t, const int32_t * pos,
                       int n_head, int n_kv, int hd, int n_ctx, float * part, float * out) {
@@ -1510,32 +1516,47 @@ int gemm_exact(int regime, int m_all) {
 #define PGEMM_LDS6 (PGEMM_LDS + 2 * 128 * 72)
 #define GEMM_MAX_ROWS 65536
 
+// The prompt products in a GEMV's order on the matrix cores (px_body): tiles
+// of 64 weight rows (SwiGLU: 32 of each matrix) x 64 positions, LDS two tiles
+// of 8 groups' codes, the rows' and the positions' fields (Q8: the group sums
+// too).
+#define PX_LDS (2 * 8 * 2 * (64 * 16 + 16) + 64 * 80 + 2 * 8 * 68 * 4)
+// Whether the exact regime takes it over the VALU GEMM. A launch costs a
+// tile's latency however few positions it holds (2.1 us per 256 columns), the
+// VALU GEMM about a fixed time per output, so the line is one on the outputs:
+// 4096 x 4096 crosses near 30 positions (32: 37 us against 42; 17: 37 against
+// 25), 4096 x 14336 near 40 (32: 114 against 92; 64: 117 against 182), 2 x
+// 14336 x 4096 below 17 (60 against 80 at 16). SML_PX_OUT overrides (tests).
+static int px_takes(int outputs, int m_all) {
+    return m_all > 16 && (long) outputs * m_all >= env_int("SML_PX_OUT", 150000);
+}
+static void px_launch(hipStream_t st, const char * base, int nbits, int swiglu, sml_kgemm * a) {
+    const int rt = swiglu ? 32 : 64;
+    const uint64_t tiles = (uint64_t) ((a->rows + rt - 1) / rt) * (uint64_t) ((a->m_all + 63) / 64);
+    if (tiles > 0x7FFFFFFFull || (uint64_t) a->m_all * (uint64_t) a->cols >= (1ull << 32))
+        hx_failf("prompt GEMM of %d rows x %d positions", a->rows, a->m_all);
+    char name[32];
+    snprintf(name, sizeof name, "%s_q%d%s", base, nbits, swiglu ? "_s" : "");
+    hx_launch(name, (unsigned) tiles, 1, 512, nbits == 8 ? PX_LDS + 8 * 68 * 4 : PX_LDS, st, a);
+}
+
 void op_gemm(hipStream_t st, const sml_kmat * tab, const sml_kmat * hk, int ngroups, int swiglu, int nbits, int rows, int cols,
              const int32_t * count, int m_all, int mt, int mmax, const int8_t * q, const float * scale,
              const int32_t * sums, float * y, const float * bias, const float * resid, int regime) {
     const int per256 = regime == GEMM_PER256;
     if (swiglu && (bias || resid)) hx_failf("SwiGLU GEMM takes no bias or residual");
     if ((uint64_t) rows * (uint64_t) cols >= (1ull << 32)) hx_failf("matrix too large for one GEMM launch");
-    if (regime == GEMM_REF) {
-        // exact mode's batched prompt: Q4 or Q8 inputs a multiple of 256
-        // wide, 16 weight rows x 64 positions per workgroup
-        if ((nbits != 4 && nbits != 8) || cols % 256 || count || ngroups != 1 || m_all < 1 ||
-            (uint64_t) m_all * cols >= (1ull << 32))
-            hx_failf("the exact batched GEMM takes one Q4 or Q8 matrix 256-aligned (%d bits, %d columns)", nbits, cols);
+    const int ref = regime == GEMM_REF;
+    if (ref && ((nbits != 4 && nbits != 8) || cols % 256 || count || ngroups != 1 || m_all < 1 || !hk))
+        hx_failf("the exact batched GEMM takes one Q4 or Q8 matrix 256-aligned (%d bits, %d columns)", nbits, cols);
+    if (ref || (regime == GEMM_EXACT && !count && ngroups == 1 && hk && px_takes(swiglu ? 2 * rows : rows, m_all))) {
         sml_kgemm a;
         memset(&a, 0, sizeof a);
-        a.mats = tab; a.nmat = swiglu ? 2 : 1; a.cols = cols; a.rows = rows;
-        a.m_all = m_all; a.mmax = mmax;
+        a.cols = cols; a.rows = rows; a.m_all = m_all;
         a.q = q; a.scale = scale; a.sums = sums; a.y = y; a.bias = bias; a.resid = resid;
-        if (hk) {
-            a.inl = 1;
-            a.m0[0] = hk[0];
-            if (swiglu) a.m0[1] = hk[1];
-        }
-        char xname[24];
-        snprintf(xname, sizeof xname, "sml_xgemm_q%d%s", nbits, swiglu ? "_s" : "");
-        hx_launch3(xname, (unsigned) ((rows + 15) / 16),
-                   (unsigned) ((m_all + 63) / 64), 1, 256, 0, st, &a);
+        a.m0[0] = hk[0];
+        if (swiglu) a.m0[1] = hk[1];
+        px_launch(st, ref ? "sml_pp_xgemm" : "sml_pp_gemm", nbits, swiglu, &a);
         return;
     }
     // the widest small-M launch: 32 rows in the exact regime (VALU), else 16

@@ -131,6 +131,9 @@ void op_attention_batch(hipStream_t st, const float * qkv, int qkv_stride, uint1
                         const float * sin_t, const int32_t * pos, int nseq, int n_head, int n_kv, int hd, int n_ctx,
                         int n_pos, float * part, float * out, int8_t * q_out, float * s_out, int32_t * u_out,
                         int causal, int exact, int q256);
+// Rows of a causal 1 launch (attending below n_pos) whose partials fit in
+// `part` floats.
+int op_attention_rows(int n_head, int n_kv, int hd, int n_ctx, int n_pos, size_t part);
 // Whether op_gemm computes every row with the GEMV's arithmetic in this regime
 // for m_all rows (the exact regime, or per-32 rows the VALU kernel takes).
 int gemm_exact(int regime, int m_all);
