@@ -159,10 +159,9 @@ int sml_hip_gemm_swiglu(const sml_hip_mat * gate, const sml_hip_mat * up, const 
 // summing each superblock's sq_g*dot_g and (mq_g-127)*sum_g in integers and
 // applying the fp32 scales once per 256 columns; the rest runs the per-group
 // kernels, which are exact on such activations (the scale repeats in every
-// group). Above 16 rows (prompt reading) Q4 runs on the prompt GEMM: tiles of
-// 128 weight rows (SwiGLU: 64) x 64 positions, the weight and activation
-// tiles staged in LDS, the same integer superblock sums; other widths run in
-// slices of 16 rows.
+// group). Above 16 rows (prompt reading) Q4 and Q6 run on the prompt GEMM:
+// tiles of 64 weight rows (SwiGLU: 32 of each matrix) x 64 or 128 positions,
+// the same integer superblock sums; other widths run in slices of 16 rows.
 // replaces sml_matvec_batch_flat4_sb and sml_rlp_matvec
 // (sml/sml-kernel.c:1414-1435,1820-1840) as batch_group dispatches them in
 // the prompt and default multi-sequence regimes (sml/sml-run.c:2090-2150)

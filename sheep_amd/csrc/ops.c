@@ -1507,13 +1507,6 @@ int gemm_exact(int regime, int m_all) {
 }
 
 #define GEMM_TILE 128            // chunks (groups) per pass: 64 lanes x GEMM_NI
-// The prompt GEMM (sml_pgemm_q4 / _q6): positions per tile, and its LDS: two
-// stages of a 128-row weight tile (144 bytes a row), a PGEMM_BM-position
-// activation tile (272 bytes a row) and the positions' scales and sums; Q6
-// adds the 2-bit plane's 128-row tile (72 bytes a row)
-#define PGEMM_BM 32
-#define PGEMM_LDS (2 * (128 * 144 + PGEMM_BM * 272 + PGEMM_BM * 8))
-#define PGEMM_LDS6 (PGEMM_LDS + 2 * 128 * 72)
 #define GEMM_MAX_ROWS 65536
 
 // The prompt products in a GEMV's order on the matrix cores (px_body): tiles
@@ -1563,21 +1556,31 @@ void op_gemm(hipStream_t st, const sml_kmat * tab, const sml_kmat * hk, int ngro
     const int msmall = regime == GEMM_EXACT ? 32 : 16;
     if (!count && m_all > msmall) {
         // prompt-sized: Q4 and Q6 with per-256 activations on the prompt MFMA
-        // GEMM (tiles of 128 rows, SwiGLU 64, x PGEMM_BM positions); anything
-        // else in slices of msmall rows through the small-M kernels
-        if (per256 && (nbits == 4 || nbits == 6) && cols % 256 == 0 && env_int("SML_PGEMM", 1)) {
-            const int rt = swiglu ? 64 : 128;
-            const uint64_t tiles = (uint64_t) ((rows + rt - 1) / rt) * (uint64_t) ((m_all + PGEMM_BM - 1) / PGEMM_BM);
+        // GEMM (ps_body); anything else in slices of msmall rows through the
+        // small-M kernels
+        if (per256 && hk && (nbits == 4 || nbits == 6) && cols % 256 == 0 && env_int("SML_PGEMM", 1)) {
+            // 128 positions a workgroup where that alone fills the chip (the
+            // weights' bytes are split for twice the positions: SwiGLU 2 x
+            // 14336 x 4096 at 128 positions 61 us against 75, at 512 226
+            // against 257), else 64 (4096 x 4096 at 256 30 against 41, at 512
+            // 48 against 53; 6144 x 4096 at 512 65 against 69)
+            const int rt = swiglu ? 32 : 64;
+            const uint64_t nrt = (uint64_t) ((rows + rt - 1) / rt);
+            int p = m_all > 64 && 4 * nrt * (uint64_t) ((m_all + 127) / 128) >= 7 * (uint64_t) hx.ncu ? 8 : 4;
+            const int fp = env_int("SML_PS_P", 0);
+            if (fp == 4 || fp == 8) p = fp;
+            const uint64_t tiles = nrt * (uint64_t) ((m_all + 16 * p - 1) / (16 * p));
             if (tiles > 0x7FFFFFFFull || (uint64_t) m_all * (uint64_t) cols >= (1ull << 32))
                 hx_failf("prompt GEMM of %d rows x %d positions", rows, m_all);
             sml_kgemm a;
             memset(&a, 0, sizeof a);
-            a.mats = tab; a.nmat = swiglu ? 2 : 1; a.cols = cols; a.rows = rows;
-            a.m_all = m_all; a.mmax = mmax;
+            a.cols = cols; a.rows = rows; a.m_all = m_all;
             a.q = q; a.scale = scale; a.sums = sums; a.y = y; a.bias = bias; a.resid = resid;
-            char pname[32];
-            snprintf(pname, sizeof pname, "sml_pgemm_q%d%s", nbits, swiglu ? "_s" : "");
-            hx_launch(pname, (unsigned) tiles, 1, 256, nbits == 6 ? PGEMM_LDS6 : PGEMM_LDS, st, &a);
+            a.m0[0] = hk[0];
+            if (swiglu) a.m0[1] = hk[1];
+            char pname[40];
+            snprintf(pname, sizeof pname, "sml_pp_sgemm_q%d%s_p%d", nbits, swiglu ? "_s" : "", p);
+            hx_launch(pname, (unsigned) tiles, 1, 256, (size_t) 2 * 16 * p * (256 + 32 + 4), st, &a);
             return;
         }
         // (the exact regime's VALU kernel takes 32 rows a weight read)

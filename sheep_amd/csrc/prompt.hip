@@ -322,3 +322,282 @@ __device__ void px_body(const sml_kgemm & a) {
 PX_KERNELS(sml_pp_gemm_q, 2, false) PX_KERNELS(sml_pp_gemm_q, 3, false) PX_KERNELS(sml_pp_gemm_q, 4, false)
 PX_KERNELS(sml_pp_gemm_q, 5, false) PX_KERNELS(sml_pp_gemm_q, 6, false) PX_KERNELS(sml_pp_gemm_q, 7, false)
 PX_KERNELS(sml_pp_gemm_q, 8, false) PX_KERNELS(sml_pp_xgemm_q, 4, true) PX_KERNELS(sml_pp_xgemm_q, 8, true)
+
+// ---------------------------------------------------------------- prompt GEMM in the superblock regime
+//
+// Y[p][r] = W.a[p] for a chunk of prompt positions p (hundreds) and every row
+// r of a Q4 or Q6 matrix, in the reference's prompt regime (sml_quantize_act_sb
+// and flat4_sb_body, sml/sml-kernel.c:115-185,1142-1190): per superblock b of
+// 256 columns the integer sums
+//     isum = sum_g sq_g * dot_g,    imin = sum_g (mq_g - 127) * sum(q_g),
+// then y = fma(isum, sd_b * s_b, y); y = fma(imin, md_b * s_b, y) in fp32 (s_b:
+// the position's activation scale of superblock b).
+//
+// Both sums run on the matrix cores whole, so the VALU touches an output once
+// per superblock and not once per group:
+//  - isum: v = sq_g * code < 2^14 is split into signed bytes, v = 256 hi + lo
+//    (lo = v's low byte as an int8, hi = (v + 128) >> 8), and the superblock's
+//    dots with hi and with lo are 4 chained v_mfma_i32_16x16x64_i8 each (|isum|
+//    < 2^31). Twice the matrix operations of one dot per group, at the full
+//    rate of the K = 64 form (the K = 32 form runs at half of it), and no
+//    multiply-add per group on the VALU.
+//  - imin: one v_mfma_f32_16x16x16_f16 over the 8 groups' sums, each as its
+//    low 6 bits and the rest (both exact in fp16), against mq_g - 127 twice;
+//    every product and partial sum is an integer below 2^24, so it is exact.
+//
+// Workgroup: 4 waves on the same 16 P positions, each on 16 weight rows of its
+// own (SwiGLU: two on gate, two on the same rows of up). A wave reads its
+// rows' planes straight into registers (16 rows x 64 bytes a load) and forms
+// hi and lo there once per superblock, for all P position tiles: lane l holds
+// row l%16 and, of 64 columns s, the 16 bytes that are its slice kq = l/16 of
+// nibble word kq + 4 (s/2): group 4 (s/2) + 2 (kq/2) + s%2, columns 16
+// (kq%2)..+15. The activation rows go to LDS as they are, copied by the memory
+// unit itself (no registers), double-buffered a superblock ahead; word w of
+// position p lies at w ^ (p % 16), so the 16 rows a wave reads at once fall
+// into different banks. The MFMA's A holds positions and B weight rows: a lane
+// owns weight row l%16 of a tile and positions 4 kq..+3.
+//
+// Bound: VALU issue, half of it used (a tile and superblock costs 24
+// instructions of epilogue, 9 MFMAs and 200 / P of splitting the weights);
+// the rest is waits of the two to four waves a SIMD holds. Against a dot per
+// group with the multiply by sq_g and a second product for the min term on
+// every group (512 positions, us): SwiGLU 2 x 14336 x 4096 364 -> 226, 4096 x
+// 14336 194 -> 142, Q6 225 -> 167; the same sums, the same bits. Two blocks of
+// rows a wave: 223 and 259. 8 waves a workgroup, three buffers and the weights
+// two superblocks ahead: 258 and 157.
+//
+// Tiles are numbered so that consecutive ones share their weight rows and sit
+// on one XCD (workgroup i runs on XCD i mod 8).
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+#define PS_STAGE(P) ((P) * 16 * (256 + 32 + 4))        // codes, group sums in fp16, scale of 16 P positions: two in LDS
+
+// 16 bytes a lane from base + off straight into LDS, the wave's 64 lanes side
+// by side from dst (a wave-uniform address) on. Written out because the
+// compiler, which cannot tell the buffers apart, otherwise waits for every copy
+// in flight before the next LDS read; the caller waits (vmcnt) and then meets
+// the other waves before any of the bytes is read. (Loads that the compiler
+// counts itself only ever wait longer for the copies it does not.)
+__device__ __forceinline__ void copy_lds16(const void * base, uint32_t off, const void * dst) {
+    const uint32_t at = (uint32_t) (uintptr_t) (const __attribute__((address_space(3))) void *) dst;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :: "s"(__builtin_amdgcn_readfirstlane(at)), "v"(off), "s"(base) : "memory");
+}
+
+template <int NB, bool SW, int P>
+__device__ void ps_body(const sml_kgemm & a) {
+    constexpr int NP = 16 * P;
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int n = a.cols, ng = n / 32, nsb = n / 256, m_all = a.m_all, rows = a.rows;
+    const int tid = threadIdx.x, lane = tid & 63, kq = lane >> 4, i16 = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr int NW = 4;                               // waves
+    constexpr int RT = SW ? 8 * NW : 16 * NW;
+    const int nrt = (rows + RT - 1) / RT, npt = (m_all + NP - 1) / NP, total = nrt * npt;
+    const int id = blockIdx.x, xcd = id & 7, slot = id >> 3, q8 = total >> 3, rem = total & 7;
+    const int lid = (xcd < rem ? xcd * (q8 + 1) : rem * (q8 + 1) + (xcd - rem) * q8) + slot;
+    const int rt = lid / npt, r0 = rt * RT, p0 = (lid - rt * npt) * NP;
+
+    // this wave's 16 weight rows (SwiGLU: waves 0 and 1 of gate, 2 and 3 the same of up)
+    constexpr int NIB = NB == 6 ? 1 : 0;
+    const bool up = SW && wave >= NW / 2;
+    const int grow = r0 + 16 * (SW ? wave & (NW / 2 - 1) : wave) + i16;
+    const sml_kmat & m = up ? a.m0[SW ? 1 : 0] : a.m0[0];
+    const size_t wr = (size_t) min(grow, rows - 1);
+    const uint8_t * wn = m.plane[NIB] + wr * (size_t) (n / 2) + 16 * kq;
+    const uint8_t * wh = m.plane[0] + wr * (size_t) (n / 4) + 16 * (kq & 1);
+    const uint8_t * fqb = m.sqmq + wr * (size_t) ng * 2;
+    const uint8_t * fdb = (const uint8_t *) m.sdmd + wr * (size_t) nsb * 4;
+    struct {
+        v4u w[2], h[2];             // the row's nibble words kq, kq + 4; Q6: its halves of the two 2-bit packs
+        uint32_t sq[2];             // (sq, mq) of groups 2 (kq/2), +1 and 4 + 2 (kq/2), +1
+        v2u mq;                     // (sq, mq) of groups 4 (kq%2)..+3
+        uint32_t fd;                // (sd, md)
+    } raw;
+    auto fetch_w = [&](int b) {
+        #pragma unroll
+        for (int p = 0; p < 2; p++) {
+            raw.w[p] = gld<v4u>(wn + (size_t) b * 128 + 64 * p);
+            if constexpr (NB == 6) raw.h[p] = gld<v4u>(wh + (size_t) b * 64 + 32 * p);
+            raw.sq[p] = gld<uint32_t>(fqb + (size_t) b * 16 + 8 * p + 4 * (kq >> 1));
+        }
+        raw.mq = gld<v2u>(fqb + (size_t) b * 16 + 8 * (kq & 1));
+        raw.fd = gld<uint32_t>(fdb + (size_t) b * 4);
+    };
+    // the positions: wave w copies rows 4 (8 i + w)..+3 of the tile, a lane 16
+    // bytes; positions past the end read the last one
+    constexpr int NC = 4 * P / NW;
+    uint32_t aoff[NC];
+    #pragma unroll
+    for (int i = 0; i < NC; i++) {
+        const int pr = 4 * (NW * i + wave) + (lane >> 4);
+        aoff[i] = (uint32_t) min(p0 + pr, m_all - 1) * (uint32_t) n + 16u * (uint32_t) ((lane & 15) ^ (pr & 15));
+    }
+    auto fetch_a = [&](int b) {
+        uint8_t * base = lds + (size_t) (b & 1) * PS_STAGE(P) + wave * 1024;
+        #pragma unroll
+        for (int i = 0; i < NC; i++) copy_lds16(a.q, aoff[i] + 256u * (uint32_t) b, base + i * (NW * 1024));
+    };
+    // the positions' group sums and scales: thread t takes 4 groups (t%2) of
+    // position t/2
+    const int sp = tid >> 1, sh = tid & 1;
+    const bool sums = tid < 2 * NP;
+    const size_t soff = (size_t) min(p0 + (sums ? sp : 0), m_all - 1) * ng + 4 * sh;
+    int4 su = make_int4(0, 0, 0, 0);
+    float ss = 0.0f;
+    auto fetch_s = [&](int b) {
+        if (sums) { su = gld<int4>(a.sums + soff + 8 * b); ss = gld<float>(a.scale + soff + 8 * b); }
+    };
+    auto stage_s = [&](int b) {
+        if (!sums) return;
+        uint8_t * base = lds + (size_t) (b & 1) * PS_STAGE(P) + NP * 256;
+        const int sv[4] = {su.x, su.y, su.z, su.w};
+        v4h lo, hi;
+        #pragma unroll
+        for (int i = 0; i < 4; i++) {
+            lo[i] = (_Float16) (float) (sv[i] & 63);
+            hi[i] = (_Float16) (float) (sv[i] & ~63);
+        }
+        *(v4h *) (base + sp * 32 + 8 * sh) = lo;
+        *(v4h *) (base + sp * 32 + 16 + 8 * sh) = hi;
+        if (sh == 0) *(float *) (base + NP * 32 + sp * 4) = ss;
+    };
+    int ao[4];                                          // the lane's words of 64 columns s in its position's row
+    #pragma unroll
+    for (int s = 0; s < 4; s++) ao[s] = i16 * 256 + 16 * ((8 * (s >> 1) + 4 * (kq >> 1) + 2 * (s & 1) + (kq & 1)) ^ i16);
+
+    float acc[P][4];
+    #pragma unroll
+    for (int u = 0; u < P; u++)
+        #pragma unroll
+        for (int r = 0; r < 4; r++) acc[u][r] = 0.0f;
+
+    auto step = [&](int b) {
+        // hi and lo of the wave's rows
+        v4i hi[4], lo[4];
+        v4h bm;
+        #pragma unroll
+        for (int s = 0; s < 4; s++) {
+            typedef unsigned short v2s __attribute__((ext_vector_type(2)));
+            const unsigned sq = (raw.sq[s >> 1] >> (16 * (s & 1))) & 0xFFu;
+            const v2s m2 = __builtin_bit_cast(v2s, sq | sq << 16), k2 = {0x80, 0x80};
+            #pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const unsigned w = raw.w[s >> 1][e] >> (4 * (s & 1));
+                unsigned c0 = w & 0x000F000Fu, c1 = (w >> 8) & 0x000F000Fu;      // columns 0, 2 and 1, 3
+                if constexpr (NB == 6) {
+                    const unsigned h = raw.h[s >> 1][e] >> (4 * (kq >> 1) + 2 * (s & 1));
+                    c0 |= (h & 0x00030003u) << 4;
+                    c1 |= ((h >> 8) & 0x00030003u) << 4;
+                }
+                const unsigned u0 = __builtin_bit_cast(unsigned, (v2s) (__builtin_bit_cast(v2s, c0) * m2 + k2));
+                const unsigned u1 = __builtin_bit_cast(unsigned, (v2s) (__builtin_bit_cast(v2s, c1) * m2 + k2));
+                hi[s][e] = (int) __builtin_amdgcn_perm(u1, u0, 0x07030501u);
+                lo[s][e] = (int) (__builtin_amdgcn_perm(u1, u0, 0x06020400u) ^ 0x80808080u);
+            }
+        }
+        #pragma unroll
+        for (int i = 0; i < 4; i++)
+            bm[i] = (_Float16) (float) ((int) ((raw.mq[i >> 1] >> (16 * (i & 1) + 8)) & 0xFFu) - 127);
+        const float dsc = h2f((uint16_t) (raw.fd & 0xFFFFu)), mdsc = h2f((uint16_t) (raw.fd >> 16));
+        const bool more = b + 1 < nsb;
+        if (more) {
+            fetch_a(b + 1);
+            fetch_s(b + 1);
+            fetch_w(b + 1);
+        }
+        const uint8_t * base = lds + (size_t) (b & 1) * PS_STAGE(P);
+        // two position tiles at a time, the hi and the lo sums apart: four
+        // independent chains of MFMAs (a chain's next product waits for its
+        // last); the next pair's operands are read during this one's epilogue
+        v4i av[2][4];
+        v4h as[2];
+        float4 s4[2];
+        auto operands = [&](int u0) {
+            #pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const int u = u0 + k;
+                #pragma unroll
+                for (int s = 0; s < 4; s++) av[k][s] = *(const v4i *) (base + u * 4096 + ao[s]);
+                as[k] = *(const v4h *) (base + NP * 256 + (16 * u + i16) * 32 + 8 * kq);
+                s4[k] = *(const float4 *) (base + NP * 288 + (16 * u + 4 * kq) * 4);
+            }
+        };
+        operands(0);
+        #pragma unroll
+        for (int u0 = 0; u0 < P; u0 += 2) {
+            const float sv[2][4] = {{s4[0].x, s4[0].y, s4[0].z, s4[0].w}, {s4[1].x, s4[1].y, s4[1].z, s4[1].w}};
+            v4i h[2], l[2];
+            v4f im[2];
+            #pragma unroll
+            for (int s = 0; s < 4; s++)
+                #pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    h[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[k][s], hi[s], s ? h[k] : v4i{0, 0, 0, 0}, 0, 0, 0);
+                    l[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[k][s], lo[s], s ? l[k] : v4i{0, 0, 0, 0}, 0, 0, 0);
+                }
+            #pragma unroll
+            for (int k = 0; k < 2; k++)
+                im[k] = __builtin_amdgcn_mfma_f32_16x16x16f16(as[k], bm, v4f{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+            if (u0 + 2 < P) operands(u0 + 2);
+            #pragma unroll
+            for (int k = 0; k < 2; k++) {
+                float (&o)[4] = acc[u0 + k];
+                #pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    o[r] += (float) ((h[k][r] << 8) + l[k][r]) * (dsc * sv[k][r]);
+                    o[r] += im[k][r] * (mdsc * sv[k][r]);
+                }
+                // (an empty statement on the sums so far: left free, the
+                // products of every tile are held in registers at once)
+                asm volatile("" : "+v"(o[0]), "+v"(o[1]), "+v"(o[2]), "+v"(o[3]));
+            }
+        }
+        if (more) stage_s(b + 1);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the next superblock's rows are in LDS
+        __syncthreads();
+    };
+    fetch_a(0);
+    fetch_s(0);
+    fetch_w(0);
+    stage_s(0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    for (int b = 0; b < nsb; b++) step(b);
+
+    if constexpr (SW) {
+        // the up waves hand their sums to the gate waves through LDS
+        float4 * x = (float4 *) lds + (wave & (NW / 2 - 1)) * P * 64 + lane;
+        if (up) {
+            #pragma unroll
+            for (int u = 0; u < P; u++) x[u * 64] = make_float4(acc[u][0], acc[u][1], acc[u][2], acc[u][3]);
+        }
+        __syncthreads();
+        if (up) return;
+        #pragma unroll
+        for (int u = 0; u < P; u++) {
+            const float4 v = x[u * 64];
+            acc[u][0] = silu_ref(acc[u][0]) * v.x;                                   // sml/sml-run.c:416-426
+            acc[u][1] = silu_ref(acc[u][1]) * v.y;
+            acc[u][2] = silu_ref(acc[u][2]) * v.z;
+            acc[u][3] = silu_ref(acc[u][3]) * v.w;
+        }
+    }
+    if (grow >= rows) return;
+    #pragma unroll
+    for (int u = 0; u < P; u++)
+        #pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int pos = p0 + 16 * u + 4 * kq + r;
+            if (pos >= m_all) continue;
+            float v = acc[u][r];
+            if (!SW && a.bias) v += a.bias[grow];
+            if (!SW && a.resid) v = a.resid[(size_t) pos * rows + grow] + v;
+            a.y[(size_t) pos * rows + grow] = v;
+        }
+}
+
+#define PS_KERNEL(NB, P)                                                                                              \
+    extern "C" __global__ __launch_bounds__(256, 2) void sml_pp_sgemm_q##NB##_p##P(const sml_kgemm a) { ps_body<NB, false, P>(a); } \
+    extern "C" __global__ __launch_bounds__(256, 2) void sml_pp_sgemm_q##NB##_s_p##P(const sml_kgemm a) { ps_body<NB, true, P>(a); }
+PS_KERNEL(4, 4) PS_KERNEL(4, 8) PS_KERNEL(6, 4) PS_KERNEL(6, 8)
