@@ -27,7 +27,9 @@ static void ing_grid(hipStream_t st, const float * wp, int rows, int cols, int g
     a.wp = wp; a.wt = wt; a.facs = facs; a.out_l = out_l; a.out_s = out_s;
     a.rows = rows; a.cols = cols; a.group = group; a.nbits = nbits; a.rem = rem;
     a.ncand = ncand; a.iters = iters; a.refit = refit;
-    const char * k = group != 32 ? "sml_ing_grid" : wt ? "sml_ing_grid32w" : "sml_ing_grid32";
+    // groups of 32 hold their codes packed: bytes up to 8 bits, halves above
+    const char * k = group != 32 ? "sml_ing_grid" : nbits > 8 ? (wt ? "sml_ing_grid32w_h" : "sml_ing_grid32_h")
+                                                              : (wt ? "sml_ing_grid32w" : "sml_ing_grid32");
     hx_launch(k, blocks((int64_t) rows * (cols / group)), 1, 256, 0, st, &a);
 }
 
@@ -249,8 +251,9 @@ int sml_hip_requant(const float * w, int rows, int cols, int nbits, const int32_
         hx_launch("sml_ing_rank", blocks(cols), (unsigned) nslice, 256, 0, 0, &k);
         hx_launch("sml_ing_scatter", blocks(cols), 1, 256, 0, 0, &k);
     }
-    sml_king_gather gth = { w, perm, wp, rows, cols };
-    hx_launch("sml_ing_gather", blocks((int64_t) nw), 1, 256, 0, 0, &gth);
+    const size_t rb = (size_t) cols * 4;
+    sml_king_gather gth = { w, perm, wp, rows, cols, rb <= 160 * 1024 };
+    hx_launch("sml_ing_gather", (unsigned) rows, 1, cols < 4096 ? 256 : 1024, gth.lds ? rb : 0, 0, &gth);
     ing_grid(0, wp, rows, cols, 32, nbits, 0, wt, dfacs, nf, 3, 1, mins, steps);
     sml_king_two t2;
     memset(&t2, 0, sizeof t2);

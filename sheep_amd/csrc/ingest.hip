@@ -107,25 +107,42 @@ extern "C" __global__ __launch_bounds__(256) void sml_ing_colfold(const sml_king
 // A stable argsort by counting: the rank of key[c] is the number of columns
 // before it in (NaN, key, column) order, counted over column slices by
 // workgroups (blockIdx.y) through LDS and added with integer atomics (the
-// total does not depend on their order); then perm[rank] = c.
+// total does not depend on their order); then perm[rank] = c. A key is a
+// magnitude or NaN, so its bits order as it does, with every NaN as the
+// largest word; against columns all before the workgroup's own an equal key
+// counts, against columns all after it does not, and only the workgroup's own
+// 256 compare columns: 14336 columns in 34 us, 176 with the comparison of
+// NaN, key and column for every pair.
+__device__ __forceinline__ uint32_t order_key(float k) { return isnan(k) ? 0xFFFFFFFFu : __builtin_bit_cast(uint32_t, k); }
+
 extern "C" __global__ __launch_bounds__(256) void sml_ing_rank(const sml_king_rank a) {
-    __shared__ float tile[1024];
-    const int c = blockIdx.x * 256 + threadIdx.x;
-    const float kc = c < a.cols ? a.key[c] : 0.0f;
-    const bool nc = isnan(kc);
-    const int j0 = blockIdx.y * a.slice, j1 = min(a.cols, j0 + a.slice);
+    __shared__ uint4 tile[64];
+    const int c = blockIdx.x * 256 + threadIdx.x, b0 = blockIdx.x * 256;
+    const uint32_t kc = c < a.cols ? order_key(a.key[c]) : 0u;
+    const int j0 = blockIdx.y * a.slice, j1 = min(a.cols, j0 + a.slice);       // slices of whole 256s
     int rank = 0;
-    for (int t0 = j0; t0 < j1; t0 += 1024) {
+    for (int t0 = j0; t0 < j1; t0 += 256) {
+        const int tn = min(256, j1 - t0);
         __syncthreads();
-        for (int j = threadIdx.x; j < 1024; j += 256) tile[j] = t0 + j < j1 ? a.key[t0 + j] : 0.0f;
+        if ((int) threadIdx.x < tn) ((uint32_t *) tile)[threadIdx.x] = order_key(a.key[t0 + threadIdx.x]);
         __syncthreads();
-        const int tn = j1 - t0 < 1024 ? j1 - t0 : 1024;
-        for (int j = 0; j < tn; j++) {
-            const float kj = tile[j];
-            const bool nj = isnan(kj);
-            // NaN keys after every number
-            const bool before = nc ? (!nj || t0 + j < c) : (!nj && (kj < kc || (kj == kc && t0 + j < c)));
-            rank += before;
+        if (t0 == b0 || tn < 256) {
+            for (int j = 0; j < tn; j++) {
+                const uint32_t kj = ((const uint32_t *) tile)[j];
+                rank += kj < kc || (kj == kc && t0 + j < c);
+            }
+        } else if (t0 < b0) {
+            #pragma unroll 8
+            for (int j = 0; j < 64; j++) {
+                const uint4 k = tile[j];
+                rank += (k.x <= kc) + (k.y <= kc) + (k.z <= kc) + (k.w <= kc);
+            }
+        } else {
+            #pragma unroll 8
+            for (int j = 0; j < 64; j++) {
+                const uint4 k = tile[j];
+                rank += (k.x < kc) + (k.y < kc) + (k.z < kc) + (k.w < kc);
+            }
         }
     }
     if (c < a.cols && rank) atomicAdd(a.cnt + c, rank);
@@ -136,49 +153,99 @@ extern "C" __global__ __launch_bounds__(256) void sml_ing_scatter(const sml_king
     if (c < a.cols) a.perm[a.cnt[c]] = c;
 }
 
-extern "C" __global__ __launch_bounds__(256) void sml_ing_gather(const sml_king_gather a) {
-    const int64_t i = (int64_t) blockIdx.x * 256 + threadIdx.x;
-    if (i >= (int64_t) a.rows * a.cols) return;
-    const int64_t r = i / a.cols;
-    a.wp[i] = a.w[r * a.cols + a.perm[i % a.cols]];
+// A workgroup per row: the row into LDS in 16-byte words, then its columns
+// from there (from memory a lane's four scattered words are four requests).
+// Rows past the LDS (a.lds 0) read them from memory.
+// 4096 x 14336: 76 us (6.2 TB/s), 333 with a 64-bit division per weight, 285
+// without it and the row in memory.
+struct __attribute__((packed, aligned(4))) int4_a4 { int x, y, z, w; };      // the caller's arrays: 4-byte aligned
+struct __attribute__((packed, aligned(4))) float4_a4 { float x, y, z, w; };
+extern "C" __global__ __launch_bounds__(1024) void sml_ing_gather(const sml_king_gather a) {
+    extern __shared__ float4 row[];
+    const float * w = a.w + (size_t) blockIdx.x * a.cols;
+    float * o = a.wp + (size_t) blockIdx.x * a.cols;
+    if (a.lds) {
+        for (int c = 4 * (int) threadIdx.x; c < a.cols; c += 4 * (int) blockDim.x) {
+            const float4_a4 v = *(const float4_a4 *) (w + c);
+            row[c / 4] = make_float4(v.x, v.y, v.z, v.w);
+        }
+        __syncthreads();
+    }
+    const float * s = (const float *) row;
+    for (int c = 4 * (int) threadIdx.x; c < a.cols; c += 4 * (int) blockDim.x) {
+        const int4_a4 p = *(const int4_a4 *) (a.perm + c);
+        *(float4 *) (o + c) = a.lds ? make_float4(s[p.x], s[p.y], s[p.z], s[p.w]) : make_float4(w[p.x], w[p.y], w[p.z], w[p.w]);
+    }
 }
 
 // ---------------------------------------------------------------- the asymmetric grid
-// Weighted error of one candidate (l, step) over the group, and (STORE) its
-// codes into q. follows sml/sml-quant.c:20-33 as the grid's vectorized loop
-// computes it: d = fma(qv, step, l) - g, then e = e + (d*d)*w in order. WT
-// false: every weight is 1 (the product by 1 is exact, so it is left out).
-template <int G, bool WT, bool STORE>
+// The searches divide every weight of a group by one step, and a correctly
+// rounded division is ten instructions against the seven of the rest of an
+// error term. With y = RN(1/step) found once (an IEEE division), a quotient is
+// five: q0 = x*y, q1 = q0 + (x - q0*step)*y, q2 = q1 + (x - q1*step)*y, each
+// residual and update one fused multiply-add. q1 is within one ulp of the
+// quotient (q0 is within 1.5, and the update leaves its own rounding and a
+// 2^-22 part of that), and then q2 is the correctly rounded quotient
+// (Markstein's theorem: y is the rounded reciprocal, q1 within an ulp, the
+// residual exact). It asks that nothing overflows and no residual underflows:
+// div_safe admits steps and values between 2^-60 and 2^60, where a quotient
+// that rounds to 0 is the only one whose residual may lose bits. Everything
+// else (NaN and infinities too) divides as before.
+__device__ __forceinline__ bool div_safe(float l, float step) {
+    return fabsf(l) < 0x1p60f && step > 0x1p-60f && step < 0x1p60f;
+}
+__device__ __forceinline__ float quot(float x, float step, float y) {
+    const float q0 = x * y;
+    const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, step, x), y, q0);
+    return __builtin_fmaf(__builtin_fmaf(-q1, step, x), y, q1);
+}
+
+// Weighted error of one candidate (l, step) over the group, and its codes
+// packed into q, CB bits each. follows sml/sml-quant.c:20-33 as the grid's
+// vectorized loop computes it: d = fma(qv, step, l) - g, then e = e + (d*d)*w
+// in order. WT false: every weight is 1 (the product by 1 is exact, so it is
+// left out). FAST: quotients through the reciprocal, nothing NaN.
+template <int G, int CB, bool WT, bool REM, bool FAST>
 __device__ __forceinline__ float err32(const float (&g)[G], const float * w, float l, float step, float n, int rem,
-                                       float (&q)[G]) {
+                                       uint32_t (&q)[G * CB / 32]) {
     float e = 0.0f;
+    const float y = FAST ? 1.0f / step : 0.0f;
     #pragma unroll
     for (int i = 0; i < G; i++) {
-        float c = __builtin_rintf((g[i] - l) / step);
-        if (c < 0.0f) c = 0.0f;
-        if (c > n) c = n;
-        if constexpr (STORE) q[i] = c;
-        const float qv = rem ? (float) ((((int) c >> rem) << rem) + (1 << (rem - 1))) : c;
+        float c;
+        if constexpr (FAST) c = __builtin_amdgcn_fmed3f(__builtin_rintf(quot(g[i] - l, step, y)), 0.0f, n);
+        else {
+            c = __builtin_rintf((g[i] - l) / step);
+            if (c < 0.0f) c = 0.0f;
+            if (c > n) c = n;
+        }
+        // a NaN code makes the error NaN, which replaces nothing: its code is not read
+        if constexpr (CB == 8) q[i / 4] = __builtin_amdgcn_cvt_pk_u8_f32(c, i & 3, i & 3 ? q[i / 4] : 0u);
+        else q[i / 2] = i & 1 ? q[i / 2] | (uint32_t) c << 16 : (uint32_t) c;
+        const float qv = REM ? (float) ((((int) c >> rem) << rem) + (1 << (rem - 1))) : c;
         const float d = __builtin_fmaf(qv, step, l) - g[i];
         e = WT ? e + (d * d) * w[i] : e + d * d;
     }
     return e;
 }
 
-// One lane per group of 32, the weights and the current codes in registers.
-// A refit's candidate codes are not kept: when it wins they are derived again
-// from its (min, step) -- the same function, so the same codes -- which
-// keeps the lane under 128 registers.
+// One lane per group of 32: the weights and the codes of the current and the
+// tried (min, step) in registers, codes packed 8 bits each (16 above 8 bits).
+// Bound by VALU issue (the order of a group's sums is serial, so the lanes
+// are the parallelism): 4096 x 14336 at 4 bits, 20 factors and 3 refits,
+// 3994 us with IEEE divisions and float codes derived again for each refit
+// that won, 1740 so.
 // follows sml/sml-quant.c:38-95 (sml_asym_grid)
-template <bool WT>
+template <int CB, bool WT, bool REM>
 __device__ __forceinline__ void grid32_body(const sml_king_grid & a) {
-    constexpr int G = 32;
+    constexpr int G = 32, NQ = G * CB / 32;
     const int ng = a.cols / G;
     const int64_t t = (int64_t) blockIdx.x * 256 + threadIdx.x;
     if (t >= (int64_t) a.rows * ng) return;
     const int j = (int) (t % ng);
     const float * gp = a.wp + (size_t) t * G;        // row r, group j: (r*ng + j)*32
-    float g[G], q[G];
+    float g[G];
+    uint32_t q[NQ], q2[NQ];
     float w[WT ? G : 1];
     #pragma unroll
     for (int i = 0; i < G; i += 4) {
@@ -190,46 +257,63 @@ __device__ __forceinline__ void grid32_body(const sml_king_grid & a) {
         for (int i = 0; i < G; i++) w[i] = a.wt[(size_t) j * G + i];
     }
     const float n = (float) ((1 << a.nbits) - 1);
-    float lo = g[0], hi = g[0], ws = 0.0f;
+    float lo = g[0], hi = g[0], ws = 0.0f, gm = 0.0f;
+    bool safe = true;
     #pragma unroll
     for (int i = 0; i < G; i++) {
         if (g[i] < lo) lo = g[i];
         if (g[i] > hi) hi = g[i];
+        safe = safe && fabsf(g[i]) < 0x1p60f;
         ws = ws + (WT ? w[i] : 1.0f);
+        gm = gm + (WT ? w[i] * g[i] : g[i]);
     }
+    gm = gm / ws;
+    // the error by reciprocals where every lane's values allow it
+    auto err = [&](float l, float step, uint32_t (&qo)[NQ]) {
+        return __any(!(safe && div_safe(l, step))) ? err32<G, CB, WT, REM, false>(g, w, l, step, n, a.rem, qo)
+                                                   : err32<G, CB, WT, REM, true>(g, w, l, step, n, a.rem, qo);
+    };
     const float c = (lo + hi) * 0.5f;
     float bl = 0.0f, bs = 0.0f, be = 0.0f;
     for (int k = 0; k < a.ncand; k++) {
         const float half = (hi - lo) * 0.5f * a.facs[k];
         float l = c - half;
         float step = fmaxf(2.0f * half, 1e-12f) / n;
-        float e = err32<G, WT, true>(g, w, l, step, n, a.rem, q);
-        if (a.refit) {
-            for (int it = 0; it < a.iters; it++) {
-                float qm = 0.0f, gm = 0.0f;
+        float e = err(l, step, q);
+        // a refit that does not win leaves the codes as they were, so the
+        // next would repeat it: the wave goes on while a lane's last one won
+        bool won = a.refit != 0;
+        for (int it = 0; it < a.iters && __any(won); it++) {
+            float qm = 0.0f;
+            if constexpr (WT) {
                 #pragma unroll
-                for (int i = 0; i < G; i++) {
-                    qm = qm + (WT ? w[i] * q[i] : q[i]);
-                    gm = gm + (WT ? w[i] * g[i] : g[i]);
-                }
-                qm = qm / ws;
-                gm = gm / ws;
-                float var = 0.0f, cov = 0.0f;
+                for (int i = 0; i < G; i++) qm = qm + w[i] * (float) (q[i * CB / 32] >> (i * CB % 32) & ((1u << CB) - 1));
+            } else {
+                // whole numbers below 2^24: the float sum in any order
+                uint32_t s = 0;
                 #pragma unroll
-                for (int i = 0; i < G; i++) {
-                    const float dq = q[i] - qm;
-                    const float wdq = WT ? w[i] * dq : dq;
-                    var = var + wdq * dq;
-                    cov = cov + wdq * (g[i] - gm);
-                }
-                float s2 = var > 1e-12f ? cov / fmaxf(var, 1e-12f) : step;
-                s2 = fmaxf(s2, 1e-12f);
-                const float l2 = __builtin_fmaf(-s2, qm, gm);
-                const float e2 = err32<G, WT, false>(g, w, l2, s2, n, a.rem, q);
-                if (e2 < e) {
-                    l = l2; step = s2; e = e2;
-                    err32<G, WT, true>(g, w, l, step, n, a.rem, q);
-                }
+                for (int i = 0; i < NQ; i++)
+                    s = CB == 8 ? __builtin_amdgcn_sad_u8(q[i], 0, s) : s + (q[i] & 0xFFFFu) + (q[i] >> 16);
+                qm = (float) s;
+            }
+            qm = qm / ws;
+            float var = 0.0f, cov = 0.0f;
+            #pragma unroll
+            for (int i = 0; i < G; i++) {
+                const float dq = (float) (q[i * CB / 32] >> (i * CB % 32) & ((1u << CB) - 1)) - qm;
+                const float wdq = WT ? w[i] * dq : dq;
+                var = var + wdq * dq;
+                cov = cov + wdq * (g[i] - gm);
+            }
+            float s2 = var > 1e-12f ? cov / fmaxf(var, 1e-12f) : step;
+            s2 = fmaxf(s2, 1e-12f);
+            const float l2 = __builtin_fmaf(-s2, qm, gm);
+            const float e2 = err(l2, s2, q2);
+            won = e2 < e;
+            if (won) {
+                l = l2; step = s2; e = e2;
+                #pragma unroll
+                for (int i = 0; i < NQ; i++) q[i] = q2[i];
             }
         }
         if (k == 0 || e < be) { bl = l; bs = step; be = e; }
@@ -238,8 +322,15 @@ __device__ __forceinline__ void grid32_body(const sml_king_grid & a) {
     a.out_s[t] = bs;
 }
 
-extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void sml_ing_grid32(const sml_king_grid a) { grid32_body<false>(a); }
-extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void sml_ing_grid32w(const sml_king_grid a) { grid32_body<true>(a); }
+#define GRID32(name, CB, WT, W)                                                                                 \
+    extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W))) void name(const sml_king_grid a) { \
+        if (a.rem) grid32_body<CB, WT, true>(a);                                                                \
+        else grid32_body<CB, WT, false>(a);                                                                     \
+    }
+GRID32(sml_ing_grid32, 8, false, 4)
+GRID32(sml_ing_grid32w, 8, true, 3)
+GRID32(sml_ing_grid32_h, 16, false, 3)
+GRID32(sml_ing_grid32w_h, 16, true, 2)
 
 // Any group that is a multiple of 8 up to 256 (gcc's 8-wide loop covers the
 // whole group, so the order is the one above), read from memory; the codes
@@ -355,7 +446,9 @@ extern "C" __global__ __launch_bounds__(256) void sml_ing_two(const sml_king_two
 }
 
 // ---------------------------------------------------------------- the field search
-// One lane per group. follows sml/sml-quant.c:101-137 (sml_field_search):
+// One lane per group; groups of 32 by the reciprocal of each step (4096 x
+// 14336, radius 2: 912 us with IEEE divisions, 395 so).
+// follows sml/sml-quant.c:101-137 (sml_field_search):
 // dd = fma(c, S, M) - g, e = fma(dd*dd, w, e) in order.
 template <int G>
 __device__ __forceinline__ void field_body(const sml_king_field & a, int64_t t, int j, const float * gp) {
@@ -381,11 +474,17 @@ __device__ __forceinline__ void field_body(const sml_king_field & a, int64_t t, 
     float be = 0.0f;
     int bs = qs0, bm = qm0;
     bool first = true;
+    bool safe = true;
+    if constexpr (G > 0) {
+        #pragma unroll
+        for (int i = 0; i < G; i++) safe = safe && fabsf(g[i]) < 0x1p60f;
+    }
     for (int da = -a.radius; da <= a.radius; da++) {
         int qs = qs0 + da;
         if (qs < 1) qs = 1;
         if (qs > a.hi) qs = a.hi;
         const float S = fmaxf((float) qs * d, 1e-12f);
+        const float y = 1.0f / S;
         for (int db = -a.radius; db <= a.radius; db++) {
             int qm = qm0 + db;
             if (qm < 0) qm = 0;
@@ -393,13 +492,22 @@ __device__ __forceinline__ void field_body(const sml_king_field & a, int64_t t, 
             const float M = ((float) qm - (float) a.moff) * m;
             float e = 0.0f;
             if constexpr (G > 0) {
-                #pragma unroll
-                for (int i = 0; i < G; i++) {
-                    float c = __builtin_rintf((g[i] - M) / S);
-                    if (c < 0.0f) c = 0.0f;
-                    if (c > (float) a.nmax) c = (float) a.nmax;
-                    const float dd = __builtin_fmaf(c, S, M) - g[i];
-                    e = __builtin_fmaf(dd * dd, wg ? wg[i] : 1.0f, e);
+                if (__any(!(safe && div_safe(M, S)))) {
+                    #pragma unroll
+                    for (int i = 0; i < G; i++) {
+                        float c = __builtin_rintf((g[i] - M) / S);
+                        if (c < 0.0f) c = 0.0f;
+                        if (c > (float) a.nmax) c = (float) a.nmax;
+                        const float dd = __builtin_fmaf(c, S, M) - g[i];
+                        e = __builtin_fmaf(dd * dd, wg ? wg[i] : 1.0f, e);
+                    }
+                } else {
+                    #pragma unroll
+                    for (int i = 0; i < G; i++) {
+                        const float c = __builtin_amdgcn_fmed3f(__builtin_rintf(quot(g[i] - M, S, y)), 0.0f, (float) a.nmax);
+                        const float dd = __builtin_fmaf(c, S, M) - g[i];
+                        e = __builtin_fmaf(dd * dd, wg ? wg[i] : 1.0f, e);
+                    }
                 }
             } else {
                 for (int i = 0; i < GG; i++) {

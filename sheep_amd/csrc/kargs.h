@@ -416,8 +416,8 @@ typedef struct { const float * part; float * key; int cols, nchunk; } sml_king_c
 // (ascending key, NaN last, ties by column); then perm[cnt[c]] = c
 typedef struct { const float * key; int32_t * cnt; int32_t * perm; int cols, slice; } sml_king_rank;
 
-// wp[r][i] = w[r][perm[i]]
-typedef struct { const float * w; const int32_t * perm; float * wp; int rows, cols; } sml_king_gather;
+// wp[r][i] = w[r][perm[i]]; lds: the row goes through LDS (4 cols bytes)
+typedef struct { const float * w; const int32_t * perm; float * wp; int rows, cols, lds; } sml_king_gather;
 
 // Per-group (min, step) of the asymmetric grid (one lane per group).
 typedef struct {
