@@ -96,3 +96,98 @@ __device__ __forceinline__ float silu_ref(float g) {
     const float sc = __builtin_bit_cast(float, ((int) r + 127) << 23);
     return g / __builtin_fmaf(p, sc, 1.0f);
 }
+
+// ---------------------------------------------------------------- reductions, activation codes
+
+__device__ __forceinline__ float wave_sum(float v) {
+    #pragma unroll
+    for (int o = 32; o; o >>= 1) v += __shfl_xor(v, o);
+    return v;
+}
+__device__ __forceinline__ float wave_max(float v) {
+    #pragma unroll
+    for (int o = 32; o; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
+    return v;
+}
+// Butterflies inside a 16-lane DPP row (quad_perm xor 1, xor 2, then the
+// half-row and row mirrors): every lane of the row ends with the row's result.
+// A swizzle (xor 16) extends them to 32 lanes.
+template <int CTRL> __device__ __forceinline__ float dpp_f(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+}
+template <int CTRL> __device__ __forceinline__ int dpp_i(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false); }
+__device__ __forceinline__ float sum16(float v) {
+    v += dpp_f<0xB1>(v); v += dpp_f<0x4E>(v); v += dpp_f<0x141>(v); v += dpp_f<0x140>(v);
+    return v;
+}
+__device__ __forceinline__ float max16(float v) {
+    v = fmaxf(v, dpp_f<0xB1>(v)); v = fmaxf(v, dpp_f<0x4E>(v)); v = fmaxf(v, dpp_f<0x141>(v)); v = fmaxf(v, dpp_f<0x140>(v));
+    return v;
+}
+__device__ __forceinline__ int isum16(int v) {
+    v += dpp_i<0xB1>(v); v += dpp_i<0x4E>(v); v += dpp_i<0x141>(v); v += dpp_i<0x140>(v);
+    return v;
+}
+// xor 16 within 32 lanes (ds_swizzle bit mode: and 0x1F, xor 0x10)
+__device__ __forceinline__ float swz16_f(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, v), 0x401F));
+}
+__device__ __forceinline__ float sum32(float v) { v = sum16(v); return v + swz16_f(v); }
+__device__ __forceinline__ float max32(float v) { v = max16(v); return fmaxf(v, swz16_f(v)); }
+__device__ __forceinline__ int isum32(int v) { v = isum16(v); return v + __builtin_amdgcn_ds_swizzle(v, 0x401F); }
+
+// Max / sum over aligned groups of 8 lanes (quad butterflies, then the half-row mirror)
+__device__ __forceinline__ float max8(float v) {
+    v = fmaxf(v, dpp_f<0xB1>(v)); v = fmaxf(v, dpp_f<0x4E>(v)); return fmaxf(v, dpp_f<0x141>(v));
+}
+__device__ __forceinline__ int isum8(int v) { v += dpp_i<0xB1>(v); v += dpp_i<0x4E>(v); return v + dpp_i<0x141>(v); }
+
+// One activation code: lrintf(v * is) clamped to +-127, where an out-of-range
+// or NaN product converts to INT_MIN as the reference's x86 build does
+// (sml/sml-kernel.c:86-106), so it clamps to -127.
+__device__ __forceinline__ int quant1(float v, float is) {
+    const float r = __builtin_rintf(v * is);
+    int t = (r >= -2147483648.0f && r < 2147483648.0f) ? (int) r : (int) 0x80000000u;
+    return t > 127 ? 127 : t < -127 ? -127 : t;
+}
+
+// The sum of squares as the reference build computes it (sml/sml-run.c:
+// 147-152, a serial loop its compiler turns into double FMAs): one lane, in
+// order. Loads run ahead of the dependent chain in blocks of 16. x is in
+// global memory or in LDS (generic loads: this is the rare fallback of the
+// checked parallel sum below).
+__device__ __noinline__ double serial_ss(const float * x, int n) {
+    double ss = 0.0;
+    int i = 0;
+    for (; i + 16 <= n; i += 16) {
+        float v[16];
+        #pragma unroll
+        for (int j = 0; j < 16; j++) v[j] = x[i + j];
+        #pragma unroll
+        for (int j = 0; j < 16; j++) ss = __builtin_fma((double) v[j], (double) v[j], ss);
+    }
+    for (; i < n; i++) { const float v = x[i]; ss = __builtin_fma((double) v, (double) v, ss); }
+    return ss;
+}
+
+// float(ss/n) of the serial chain above, from a sum of the same squares taken
+// in any order. Every square is exact in double (24-bit mantissas), all are
+// nonnegative, so each order's sum lies within (n-1)*2^-53*(1+2^-30) of the
+// exact sum, relatively: the serial and the given sum differ by less than
+// d = 4*(n+4)*2^-53*s, with a margin for the rounding of d itself. Division
+// by n and the float conversion are monotone, so when s-d and s+d give the
+// same float that float is the serial chain's; it fails for about one input
+// in 10^4 (a rounding boundary inside the window) and for inf/NaN sums, and
+// the caller then runs the chain.
+__device__ __forceinline__ bool ss_mean_alike(double s, int n, float & out) {
+    const double d = s * ((double) (4 * (n + 4)) * 0x1p-53);
+    const float lo = (float) ((s - d) / (double) n), hi = (float) ((s + d) / (double) n);
+    out = lo;
+    return lo == hi;
+}
+
+// Four values' squares added to a double sum, in sml_normq2's order (its
+// callers share it so that their sums agree bit for bit).
+__device__ __forceinline__ double ss_add4(double ss, float4 v) {
+    return ss + ((double) v.x * v.x + (double) v.y * v.y + (double) v.z * v.z + (double) v.w * v.w);
+}

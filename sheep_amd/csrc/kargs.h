@@ -167,9 +167,11 @@ typedef struct {
     // merges that head's query heads as sml_attn_merge does and resets the
     // counter, so no merge launch follows. One launch at a time per array.
     int * cnt;
-    // sml_attnf (prompt flash form): KV positions per split (grid z), a
+    // sml_pp_flash (prompt flash form): KV positions per split (grid z), a
     // multiple of 64
     int fchunk;
+    // pos NULL (sml_ropekv, sml_pp_flash): entry b is at position pos0 + b
+    int pos0;
     // query-head subsets per kv head (the 8-wave kernels; 0 or 1: none):
     // grid y = n_kv * nsub, workgroup y takes kv head y / nsub and its query
     // heads (y % nsub) * REP .. +REP-1 (REP = n_head / n_kv / nsub)

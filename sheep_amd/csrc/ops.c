@@ -9,6 +9,11 @@
 #include "sml-hip.h"
 #include "ssf.h"
 
+static int env_int(const char * name, int dflt) {
+    const char * e = getenv(name);
+    return e && *e ? atoi(e) : dflt;
+}
+
 static size_t al256(size_t x) { return (x + 255u) & ~(size_t) 255u; }
 
 // the split-K sums op_gemm left for the next normq (ops_defer_ksum)
@@ -554,11 +559,6 @@ int sml_hip_normq(float * x, const float * resid, const float * w, float eps, in
     return 0;
 }
 
-static int env_int(const char * name, int dflt) {
-    const char * e = getenv(name);
-    return e && *e ? atoi(e) : dflt;
-}
-
 // Shape of a GEMV launch: NI chunks per lane (enough that one pass covers a
 // row: ng <= 64*NI, at most 8; SwiGLU and the fused prologue at most 4 and 2),
 // RB rows per wave (more rows per wave for tall matrices, so ~2048+ waves
@@ -959,9 +959,29 @@ void op_attention(hipStream_t st, const float * q, const float * k, const float 
     if (!cnt) hx_launch(hd == 64 ? "sml_attn_merge_d64" : "sml_attn_merge", (unsigned) n_head, 1, (unsigned) hd, 0, st, &a);
 }
 
-// LDS of the prompt flash attention (sml_attnf): two stages of a 64-position
-// K tile (272 bytes a row) and its V transposed (128 dims x 144 bytes)
-#define ATTNF_LDS (2 * (64 * 272 + 128 * 144))
+// LDS of the prompt flash attention (sml_pp_flash): two stages of 64 positions' K and V rows
+#define PF_LDS (2 * 2 * 64 * 256)
+// Prompt attention on the matrix cores (head_dim 128, K and V written): 128
+// (entry, head) rows of a kv head a workgroup, the KV range cut into splits
+// only as far as the grid lacks two workgroups per CU (then merged); splits of
+// a multiple of 64 positions, at most the partials' ceil(n_ctx / 128), and
+// none of fewer than 256: a split adds the merge and a start of ~6 us, a
+// workgroup alone on a CU takes 2 us a block. Kernel + merge in us (32 heads
+// over 8), splits 1 / 4 / 8 / 16 / 32: 64 rows at 3968 126 / 44 / 30 / 24 / 28,
+// 509 at 1531 - / 47 / 62 / - / -, 128 at 0 11.7 / 14 / 16 / 19 / 26, 2048 at 0
+// 93 / 125 / 167 / 355 / 588. SML_PF_NS forces a count.
+static void prompt_flash(hipStream_t st, sml_kattn * a, int n_ctx, int n_pos) {
+    const int rows = a->nseq * (a->n_head / a->n_kv), nqb = (rows + 127) / 128, maxs = (n_ctx + 127) / 128;
+    int ns = 1;
+    while (ns < maxs && 256 * ns < n_pos && (long) nqb * a->n_kv * ns < 2L * hx.ncu) ns++;
+    const int es = env_int("SML_PF_NS", 0);
+    if (es > 0 && es <= maxs) ns = es;
+    a->nsplit = ns;
+    a->fchunk = ((n_pos + ns - 1) / ns + 63) / 64 * 64;
+    hx_launch3("sml_pp_flash", (unsigned) a->n_kv, (unsigned) nqb, (unsigned) ns, 512, PF_LDS, st, a);
+    if (ns > 1) hx_launch("sml_pp_merge", (unsigned) (((size_t) a->nseq * a->n_head + 7) / 8), 1, 256, 0, st, a);
+}
+
 void op_attention_batch(hipStream_t st, const float * qkv, int qkv_stride, uint16_t * const * kc_slots,
                         uint16_t * const * vc_slots, const int32_t * slot, size_t layer_off, const float * cos_t,
                         const float * sin_t, const int32_t * pos, int nseq, int n_head, int n_kv, int hd, int n_ctx,
@@ -1010,20 +1030,8 @@ void op_attention_batch(hipStream_t st, const float * qkv, int qkv_stride, uint1
     a.tpw = causal ? env_int("SML_ATTN_TPW", 16) : 1;
     if (a.tpw < 1 || a.tpw > 16) a.tpw = 1;
     if (causal == 2 && env_int("SML_ATTN_FLASH", 1)) {
-        // MFMA flash form: 16 entries x one kv head per workgroup (a wave per
-        // query head), the KV range cut into splits only as far as the grid
-        // needs workgroups (then merged); splits of a multiple of 64
-        // positions, at most the partial buffer's ceil(n_ctx / 128)
         if (q_out) hx_failf("flash prompt attention does not quantize its output");
-        const int rep = n_head / n_kv, nqb = (nseq + 15) / 16;
-        const int maxs = (n_ctx + 127) / 128;
-        int ns = 1;
-        while (ns * 2 <= maxs && ns < 64 && (long) nqb * n_kv * ns < 2L * hx.ncu) ns *= 2;
-        a.nsplit = ns;
-        a.fchunk = ((n_ctx + ns - 1) / ns + 63) / 64 * 64;
-        snprintf(name, sizeof name, "sml_attnf_r%d", rep);
-        hx_launch3(name, (unsigned) nqb, (unsigned) n_kv, (unsigned) ns, (unsigned) (64 * rep), ATTNF_LDS, st, &a);
-        if (ns > 1) hx_launch3("sml_attn_merge", (unsigned) n_head, 1, (unsigned) nseq, (unsigned) hd, 0, st, &a);
+        prompt_flash(st, &a, n_ctx, n_pos);
         return;
     }
     if (causal == 2) {
@@ -1112,6 +1120,20 @@ int sml_hip_attention_prompt(const float * qkv, int n_rows, int pos0, uint16_t *
         hx_failf("prompt attention shape (heads %d/%d, head_dim %d) not supported", n_head, n_kv, hd);
     if (n_rows < 1 || n_rows > 65535 || pos0 < 0 || pos0 + n_rows > n_ctx)
         hx_failf("prompt attention over positions %d..%d of %d", pos0, pos0 + n_rows - 1, n_ctx);
+    if (hd == 128 && env_int("SML_ATTN_FLASH", 1)) {
+        // one cache, consecutive positions: nothing to look up on the device
+        sml_kattn a;
+        memset(&a, 0, sizeof a);
+        a.q = qkv; a.k = qkv + (size_t) n_head * hd; a.v = a.k + (size_t) n_kv * hd;
+        a.qkv_stride = (n_head + 2 * n_kv) * hd; a.kcache = kcache; a.vcache = vcache; a.cos_t = cos_t; a.sin_t = sin_t;
+        a.pos0 = pos0; a.part = part; a.out = out; a.n_head = n_head; a.n_kv = n_kv; a.nseq = n_rows;
+        a.inv = 1.0f / __builtin_sqrtf((float) hd);
+        hx_launch("sml_ropekv", (unsigned) n_rows, 1, (unsigned) (hd / 8 * n_kv), 0, 0, &a);
+        prompt_flash(0, &a, n_ctx, pos0 + n_rows);
+        HX(hipDeviceSynchronize());
+        HX_LEAVE();
+        return 0;
+    }
     // device tables: the one sequence's cache pointers, every row's slot (0)
     // and position
     const size_t tb = 2 * sizeof(void *) + (size_t) n_rows * 8;

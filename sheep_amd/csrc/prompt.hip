@@ -601,3 +601,289 @@ __device__ void ps_body(const sml_kgemm & a) {
     extern "C" __global__ __launch_bounds__(256, 2) void sml_pp_sgemm_q##NB##_p##P(const sml_kgemm a) { ps_body<NB, false, P>(a); } \
     extern "C" __global__ __launch_bounds__(256, 2) void sml_pp_sgemm_q##NB##_s_p##P(const sml_kgemm a) { ps_body<NB, true, P>(a); }
 PS_KERNEL(4, 4) PS_KERNEL(4, 8) PS_KERNEL(6, 4) PS_KERNEL(6, 8)
+
+// ---------------------------------------------------------------- prompt attention on MFMA (flash form)
+//
+// For prompt reading at level 2 (and the attention entry point): the entries
+// of a launch are consecutive positions of one sequence whose K and V rows
+// sml_ropekv has already rotated and written to the cache (fp16). The
+// (entry, query head) pairs of a kv head are its rows, whatever the heads a
+// kv head serves: a workgroup takes 128 of them, 16 a wave, and walks the KV
+// positions of its split in blocks of 64 with an online softmax, on
+// v_mfma_f32_16x16x32_f16 (lane l: A row / B column l%16, k = 8(l/16)..+7; D
+// rows 4(l/16)..+3 of column l%16):
+//  - S^T = K Q^T: A = the block's K rows, B = the wave's rotated q (as rope8
+//    rotates it) as two fp16 parts, q_hi = fp16(q) and q_lo = fp16(q - q_hi),
+//    so the scores carry q to ~2^-22; a lane then holds row l%16 at KV
+//    positions 4(l/16)..+3 of each 16-position tile;
+//  - the softmax in base 2 and fp32, masked past each entry's position;
+//  - O += P V: A = P straight from the S^T layout (the MFMA's k slots
+//    8(l/16)..+7 hold KV rows 4(l/16)..+3 of two 16-position tiles), as fp16
+//    high and low parts like q (P rounded once to fp16, against a sum of the
+//    unrounded P, moved a MoE prompt enough to flip a routed expert), B = V
+//    by transposing LDS reads (ds_read_b64_tr_b16: 16 lanes read 4 rows of
+//    16 dims and take a dim's 4 rows each), the same slot order.
+// K and V go from memory to LDS without registers, a block ahead, 16-byte
+// words swizzled by row so that both kinds of read touch every bank once; 4
+// waves per SIMD (two workgroups per CU). What bounds it: matrix and vector
+// instructions of the same waves (64 MFMA of 16 clocks and ~220 others a
+// block), about half of the time each. 509 rows at 1531, 32 heads over 8:
+// 40 us, 124 with a wave per head, V transposed by 2-byte LDS writes (8 to
+// a bank) and 2 waves per SIMD; 16 rows to a wave 42 against 45 for 32 (half
+// the LDS reads, half the waves).
+// One split: the output is written directly; several: partials of sml_attn's
+// layout, merged by sml_pp_merge. fp32 accumulation in its own order: graded
+// as level-2 prompt reading is.
+typedef short v4s __attribute__((ext_vector_type(4)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+#define PF_KB 64                                        // KV positions a block
+#define PF_STAGE (2 * PF_KB * 256)                      // its K rows, then its V rows
+
+__device__ void pf_body(const sml_kattn & a) {
+    constexpr int W = 8, QT = 1, HD = 128, RW = 16 * QT;               // rows (query, head) of a wave
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, i16 = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kh = blockIdx.x, rep = a.n_head / a.n_kv, nrow = a.nseq * rep;
+    const int rb = (int) (gridDim.y - 1 - blockIdx.y) * W * RW, rw = rb + wave * RW;
+    const int kvd = a.n_kv * HD, half = HD / 2;
+    auto entry = [&](int row) { return min(row, nrow - 1) / rep; };
+    auto at = [&](int b) { return a.pos ? a.pos[b] : a.pos0 + b; };
+    // this split's KV range, cut at the workgroup's last position, and the wave's end in it
+    const int t_lo = blockIdx.z * a.fchunk, t_end = min(t_lo + a.fchunk, at(entry(rb + W * RW - 1)) + 1);
+    const int w_end = rw < nrow ? min(t_end, at(entry(rw + RW - 1)) + 1) : 0;
+    const size_t sl_off = a.kc_slots ? a.layer_off : 0;
+    const uint16_t * kc = (a.kc_slots ? a.kc_slots[a.slot[entry(rb)]] : a.kcache) + sl_off + (size_t) kh * HD;
+    const uint16_t * vc = (a.vc_slots ? a.vc_slots[a.slot[entry(rb)]] : a.vcache) + sl_off + (size_t) kh * HD;
+
+    // the rotated q of each tile's row i16, dims 32c + 8g + e, as fp16 B operands (hi, lo)
+    const float sl = a.inv * 1.44269504088896341f;
+    v8h qb[QT][4], ql[QT][4];
+    int posq[QT];
+    #pragma unroll
+    for (int u = 0; u < QT; u++) {
+        const int row = min(rw + 16 * u + i16, nrow - 1), b = row / rep, h = kh * rep + (row - b * rep);
+        posq[u] = at(b);
+        const float * qp = a.q + (size_t) b * a.qkv_stride + (size_t) h * HD + 8 * g;
+        float x[4][8];
+        #pragma unroll
+        for (int c = 0; c < 4; c++)
+            #pragma unroll
+            for (int e = 0; e < 8; e += 4) *(float4 *) &x[c][e] = *(const float4 *) (qp + 32 * c + e);
+        #pragma unroll
+        for (int c = 0; c < 2; c++) {
+            float cs[8], sn[8];
+            #pragma unroll
+            for (int e = 0; e < 8; e += 4) {
+                *(float4 *) &cs[e] = *(const float4 *) (a.cos_t + (size_t) posq[u] * half + 32 * c + 8 * g + e);
+                *(float4 *) &sn[e] = *(const float4 *) (a.sin_t + (size_t) posq[u] * half + 32 * c + 8 * g + e);
+            }
+            #pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float lo = x[c][e], hi = x[c + 2][e];
+                x[c][e] = __builtin_fmaf(lo, cs[e], -(hi * sn[e]));              // sml/sml-run.c:363-368, fused as its build does
+                x[c + 2][e] = __builtin_fmaf(lo, sn[e], hi * cs[e]);
+            }
+        }
+        #pragma unroll
+        for (int c = 0; c < 4; c++)
+            #pragma unroll
+            for (int e = 0; e < 8; e++) {
+                qb[u][c][e] = (_Float16) x[c][e];
+                ql[u][c][e] = (_Float16) (x[c][e] - (float) qb[u][c][e]);
+            }
+    }
+    float m_run[QT];                                    // of row i16 of each tile (the same in its 4 lanes)
+    float l_run[QT];                                    // the lane's positions' share of its sum
+    v4f o[QT][8];
+    #pragma unroll
+    for (int u = 0; u < QT; u++) {
+        m_run[u] = -INFINITY;
+        l_run[u] = 0.0f;
+        #pragma unroll
+        for (int dt = 0; dt < 8; dt++) o[u][dt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+
+    // a block's rows into LDS: 16-byte word w of row r at place w ^ 2(r & 7);
+    // rows past the range repeat its first
+    auto fetch = [&](int buf, int t0) {
+        uint8_t * st = lds + buf * PF_STAGE;
+        const uint16_t * kb = kc + (size_t) t0 * kvd, * vb = vc + (size_t) t0 * kvd;
+        #pragma unroll
+        for (int i = 0; i < 16 / W; i++) {
+            const int r = 4 * (W * i + wave) + g;
+            const uint32_t off = (uint32_t) (t0 + r < t_end ? r : 0) * (uint32_t) (kvd * 2) + 16u * (uint32_t) (i16 ^ (2 * (r & 7)));
+            copy_lds16(kb, off, st + 4 * (W * i + wave) * 256);
+            copy_lds16(vb, off, st + PF_KB * 256 + 4 * (W * i + wave) * 256);
+        }
+    };
+    const int krow = i16 * 256, kx = 2 * (i16 & 7);     // K row i16 of a tile
+    const int vrow = 4 * g + (i16 >> 2), vx = vrow & 7; // the V row this lane reads for its 16 lanes
+    const int vat = PF_KB * 256 + vrow * 256 + 8 * (i16 & 3);
+
+    auto compute = [&](int buf, int t0) {
+        const uint8_t * st = lds + buf * PF_STAGE;
+        // S^T: 4 tiles of 16 positions x 16 rows
+        v4f s[QT][4];
+        #pragma unroll
+        for (int j = 0; j < 4; j++) {
+            #pragma unroll
+            for (int u = 0; u < QT; u++) s[u][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            #pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const v8h ka = *(const v8h *) (st + 16 * j * 256 + krow + 16 * ((4 * c + g) ^ kx));
+                #pragma unroll
+                for (int u = 0; u < QT; u++) {
+                    s[u][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qb[u][c], s[u][j], 0, 0, 0);
+                    s[u][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, ql[u][c], s[u][j], 0, 0, 0);
+                }
+            }
+        }
+        v8h pa[QT][2], pl[QT][2];
+        #pragma unroll
+        for (int u = 0; u < QT; u++) {
+            // mask (the blocks that reach past a row's position) and the block's max for the lane's row
+            const int lim = min(posq[u], t_end - 1) - t0 - 4 * g;
+            if (__any(lim < 48 + 3)) {
+                #pragma unroll
+                for (int j = 0; j < 4; j++)
+                    #pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        if (16 * j + r > lim) s[u][j][r] = -INFINITY;
+            }
+            float mx = -INFINITY;
+            #pragma unroll
+            for (int j = 0; j < 4; j++)
+                #pragma unroll
+                for (int r = 0; r < 4; r++) mx = fmaxf(mx, s[u][j][r]);
+            mx *= sl;
+            // the base of the weights is 7 below the max (weights up to 128, so
+            // that fewer low parts fall below fp16's normal range) and moves
+            // only when the max has passed it by 15 (weights up to 2^15, within
+            // the range): most blocks need no reduction over the row's lanes
+            if (__any(mx > m_run[u] + 15.0f)) {
+                mx = fmaxf(mx, __shfl_xor(mx, 16));
+                mx = fmaxf(mx, __shfl_xor(mx, 32));
+                const float m_new = mx > m_run[u] + 15.0f ? mx - 7.0f : m_run[u];
+                // rescale O (its rows are 4g..4g+3)
+                const float alpha = __builtin_amdgcn_exp2f(m_run[u] - (m_new == -INFINITY ? 0.0f : m_new));
+                l_run[u] *= alpha;
+                float al[4];
+                #pragma unroll
+                for (int r = 0; r < 4; r++) al[r] = __shfl(alpha, 4 * g + r);
+                #pragma unroll
+                for (int dt = 0; dt < 8; dt++)
+                    #pragma unroll
+                    for (int r = 0; r < 4; r++) o[u][dt][r] *= al[r];
+                m_run[u] = m_new;
+            }
+            const float mu = m_run[u] == -INFINITY ? 0.0f : m_run[u];   // no position yet: keep zeros
+            float ls = 0.0f;
+            #pragma unroll
+            for (int j = 0; j < 4; j++)
+                #pragma unroll
+                for (int r = 0; r < 4; r += 2) {
+                    const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u][j][r], sl, -mu));
+                    const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u][j][r + 1], sl, -mu));
+                    ls += p0;
+                    ls += p1;
+                    const v2h ph = {(_Float16) p0, (_Float16) p1};
+                    float r0, r1;                             // p - hi, exact
+                    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r0) : "v"(ph), "v"(p0));
+                    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r1) : "v"(ph), "v"(p1));
+                    const v2h pr = {(_Float16) r0, (_Float16) r1};
+                    pa[u][j >> 1][4 * (j & 1) + r] = ph[0];
+                    pa[u][j >> 1][4 * (j & 1) + r + 1] = ph[1];
+                    pl[u][j >> 1][4 * (j & 1) + r] = pr[0];
+                    pl[u][j >> 1][4 * (j & 1) + r + 1] = pr[1];
+                }
+            l_run[u] += ls;
+        }
+        // O += P V: per 32 positions k, slots 8g..8g+3 are rows 4g..4g+3 of
+        // tile 2k, 8g+4..8g+7 those of tile 2k+1
+        #pragma unroll
+        for (int dt = 0; dt < 8; dt++) {
+            const uint8_t * vr = st + vat + ((dt ^ vx) << 5);
+            #pragma unroll
+            for (int k = 0; k < 2; k++) {
+                typedef __attribute__((address_space(3))) v4s lv4s;
+                const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lv4s *) (vr + 32 * k * 256));
+                const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lv4s *) (vr + (32 * k + 16) * 256));
+                const v8h w = __builtin_bit_cast(v8h, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                #pragma unroll
+                for (int u = 0; u < QT; u++) {
+                    o[u][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[u][k], w, o[u][dt], 0, 0, 0);
+                    o[u][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl[u][k], w, o[u][dt], 0, 0, 0);
+                }
+            }
+        }
+    };
+
+    if (t_lo < t_end) {
+        fetch(0, t_lo);
+        int buf = 0;
+        for (int t0 = t_lo; t0 < t_end; t0 += PF_KB, buf ^= 1) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // this block's rows are in LDS
+            __syncthreads();
+            if (t0 + PF_KB < t_end) fetch(buf ^ 1, t0 + PF_KB);  // past the barrier: nobody reads the last block
+            if (t0 < w_end) compute(buf, t0);
+        }
+    }
+
+    // the lane's rows: 4g..4g+3 of each tile, dims 16dt + i16
+    const bool one = gridDim.z == 1;
+    #pragma unroll
+    for (int u = 0; u < QT; u++) {
+        l_run[u] += __shfl_xor(l_run[u], 16);
+        l_run[u] += __shfl_xor(l_run[u], 32);
+        #pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const float lq = __shfl(l_run[u], 4 * g + r), mq = __shfl(m_run[u], 4 * g + r);
+            const int row = rw + 16 * u + 4 * g + r;
+            if (row >= nrow) continue;
+            const int b = row / rep, h = kh * rep + (row - b * rep);
+            if (one) {
+                float * out = a.out + (size_t) b * a.n_head * HD + (size_t) h * HD;
+                #pragma unroll
+                for (int dt = 0; dt < 8; dt++) out[16 * dt + i16] = o[u][dt][r] / lq;
+            } else {
+                float * blk = a.part + (size_t) b * a.n_head * a.nsplit * (HD + 2);
+                float * po = blk + ((size_t) h * a.nsplit + blockIdx.z) * HD;
+                float2 * pml = (float2 *) (blk + (size_t) a.n_head * a.nsplit * HD) + (size_t) h * a.nsplit + blockIdx.z;
+                #pragma unroll
+                for (int dt = 0; dt < 8; dt++) po[16 * dt + i16] = o[u][dt][r];
+                if (i16 == 0) *pml = make_float2(mq, lq);
+            }
+        }
+    }
+}
+
+extern "C" __global__ __launch_bounds__(512, 4) void sml_pp_flash(const sml_kattn a) { pf_body(a); }
+
+// The splits of sml_pp_flash merged: 32 lanes a (row, head), four dims a lane,
+// the splits in order. A launch per head and row as the decode merge makes
+// is bound by its workgroups' start and one serial chain of loads: 509 rows
+// of 32 heads, 4 splits, 15.6 us there and 7.3 here.
+extern "C" __global__ __launch_bounds__(256) void sml_pp_merge(const sml_kattn a) {
+    const int idx = blockIdx.x * 8 + (threadIdx.x >> 5), l = threadIdx.x & 31, ns = a.nsplit;
+    if (idx >= a.nseq * a.n_head) return;
+    const int b = idx / a.n_head, h = idx - b * a.n_head;
+    const float * blk = a.part + (size_t) b * a.n_head * ns * 130;
+    const float4 * po = (const float4 *) (blk + (size_t) h * ns * 128) + l;
+    const float2 * pml = (const float2 *) (blk + (size_t) a.n_head * ns * 128) + (size_t) h * ns;
+    float M = -INFINITY;
+    for (int s = l; s < ns; s += 32) M = fmaxf(M, pml[s].x);
+    M = max32(M);                                             // finite: a row's first split is active
+    float L = 0.0f;
+    float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    #pragma unroll 4
+    for (int s = 0; s < ns; s++) {
+        const float2 ml = pml[s];
+        const float4 v = po[s * 32];
+        const float e = __builtin_amdgcn_exp2f(ml.x - M);     // 0 for splits past the position
+        L += e * ml.y;
+        o.x += e * v.x; o.y += e * v.y; o.z += e * v.z; o.w += e * v.w;
+    }
+    *((float4 *) (a.out + (size_t) idx * 128) + l) = make_float4(o.x / L, o.y / L, o.z / L, o.w / L);
+}
