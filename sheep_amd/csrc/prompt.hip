@@ -887,3 +887,89 @@ extern "C" __global__ __launch_bounds__(256) void sml_pp_merge(const sml_kattn a
     }
     *((float4 *) (a.out + (size_t) idx * 128) + l) = make_float4(o.x / L, o.y / L, o.z / L, o.w / L);
 }
+
+// ---------------------------------------------------------------- normalization + quantization of many rows
+//
+// sml_normq2's codes, scales and sums bit for bit (its sum of squares order,
+// its formulas), a workgroup a row. There each of a row's n/256 workgroups
+// reads the whole row for the norm, and every value comes by its own gather
+// from memory; here the row is read once, normalized into LDS, and each
+// output gathers from there four columns a lane (a group of 32 is 8 lanes, a
+// superblock one wave).
+// 512 x 4096 with its norm: 9.1 us, 18.6 there (mean over a layer's four).
+struct __attribute__((packed, aligned(4))) int4_a4 { int x, y, z, w; };
+struct __attribute__((packed, aligned(4))) float4_a4 { float x, y, z, w; };
+extern "C" __global__ __launch_bounds__(256) void sml_pp_normq(const sml_knormq2 a) {
+    extern __shared__ __align__(16) float y[];                // [n]
+    __shared__ double red[4];
+    const int n = a.n, tid = threadIdx.x;
+    const size_t bo = (size_t) blockIdx.x * n, bg = (size_t) blockIdx.x * (n / 32);
+    const float * x = a.x + bo;
+    if (a.norm_w) {
+        double ss = 0.0;
+        #pragma unroll 4
+        for (int i = tid * 4; i < n; i += 1024) {
+            const float4 v = *(const float4 *) (x + i);
+            *(float4 *) (y + i) = v;
+            ss = ss_add4(ss, v);
+        }
+        #pragma unroll
+        for (int o = 32; o; o >>= 1) ss += __shfl_xor(ss, o);
+        if ((tid & 63) == 0) red[tid >> 6] = ss;
+        __syncthreads();
+        const double tot = red[0] + red[1] + red[2] + red[3];
+        float msq = (float) (tot / (double) n);
+        if (a.exact && !ss_mean_alike(tot, n, msq)) {
+            // the serial chain (the same decision in every thread)
+            __syncthreads();
+            if (tid == 0) red[0] = serial_ss(x, n);
+            __syncthreads();
+            msq = (float) (red[0] / (double) n);
+        }
+        const float sc = 1.0f / sqrtf(msq + a.eps);
+        #pragma unroll 4
+        for (int i = tid * 4; i < n; i += 1024) {             // the thread's own words
+            float4 v = *(const float4 *) (y + i);
+            const float4_a4 w = *(const float4_a4 *) (a.norm_w + i);
+            v.x = v.x * sc * w.x; v.y = v.y * sc * w.y; v.z = v.z * sc * w.z; v.w = v.w * sc * w.w;
+            *(float4 *) (y + i) = v;
+        }
+    } else {
+        #pragma unroll 4
+        for (int i = tid * 4; i < n; i += 1024) *(float4 *) (y + i) = *(const float4 *) (x + i);
+    }
+    __syncthreads();
+    for (int o = 0; o < a.nout; o++) {
+        const int32_t * perm = a.perm[o];
+        #pragma unroll 4
+        for (int j0 = 0; j0 < n; j0 += 1024) {
+            const int j = j0 + 4 * tid;
+            const bool ok = j < n;                            // whole groups of 32
+            float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (ok) {
+                if (perm) {
+                    const int4_a4 p = *(const int4_a4 *) (perm + j);
+                    v[0] = y[p.x]; v[1] = y[p.y]; v[2] = y[p.z]; v[3] = y[p.w];
+                } else {
+                    *(float4 *) v = *(const float4 *) (y + j);
+                }
+            }
+            const float m4 = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+            const float amax = a.per256 ? wave_max(m4) : max8(m4);
+            const float s = amax / 127.0f;
+            const float is = s > 0.0f ? 1.0f / s : 0.0f;
+            uint32_t w = 0;
+            int t4 = 0;
+            #pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int t = quant1(v[e], is);
+                t4 += t;
+                w |= (uint32_t) (t & 0xFF) << (8 * e);
+            }
+            const int sum = isum8(t4);
+            if (!ok) continue;
+            *(uint32_t *) (a.q[o] + bo + j) = w;
+            if ((tid & 7) == 0) { a.scale[o][bg + (j >> 5)] = s; a.sums[o][bg + (j >> 5)] = sum; }
+        }
+    }
+}

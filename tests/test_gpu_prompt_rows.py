@@ -1,6 +1,8 @@
 """Prompt rows: the matrix-core attention (sml_pp_flash, sml_pp_merge) against
 float64 at the edges of its 128-row tiles, 64-position blocks and splits, over
-scores whose maximum climbs, falls or stays far below zero."""
+scores whose maximum climbs, falls or stays far below zero; and the
+row-a-workgroup normalization + quantization (sml_pp_normq, from 128 rows)
+against the form that fewer rows take, bit for bit."""
 import numpy as np
 import pytest
 
@@ -61,3 +63,34 @@ def test_flash_rows_against_float64(heads, kv, n, pos0, n_ctx, kind):
         # random sign (about 2^-21 of its terms); a weight by that and its
         # own two parts (2^-21); both move the output by their share of max |V|
         assert np.abs(got[:, h] - want).max() <= (8.0 + S) * 2.0 ** -20 * np.abs(V[:T]).max(), h
+
+
+def _read(path, cuts, ids, level, exact, vocab):
+    d = sa.Decoder(path, n_ctx=512, exact=exact)
+    try:
+        d.prompt_mode(level)
+        for a, b in zip(cuts, cuts[1:]):
+            out = d.prefill(ids[a:b], a, vocab)
+        return out, d.step(int(np.argmax(out)), len(ids), vocab)
+    finally:
+        d.close()
+
+
+@pytest.mark.parametrize("level,exact", [(1, False), (1, True), (2, False)])
+@pytest.mark.parametrize("n_embd,n_head,kv,n_ff", [(384, 3, 1, 1280), (1024, 8, 1, 1152), (2304, 18, 6, 2304)])
+def test_many_rows_quantize_as_few(tmp_path, monkeypatch, n_embd, n_head, kv, n_ff, level, exact):
+    # 128 rows and more in one read against reads of 100: the products and the
+    # wave-per-position attention do not depend on the cut
+    if exact and (n_ff % 256 or n_embd % 256):
+        pytest.skip("exact mode batches 256-aligned products")
+    monkeypatch.setenv("SML_ATTN_FLASH", "0")
+    monkeypatch.setenv("SML_PX_OUT", "0")
+    p = tmp_path / "m.ssf"
+    sa.synth_model(p, n_layer=2, n_vocab=600, nbits=4, random_perm=True, seed=n_embd, n_embd=n_embd, n_head=n_head,
+                   n_head_kv=kv, n_ff=n_ff)
+    ids = np.random.default_rng(n_ff).integers(0, 600, 200).astype(np.int32)
+    a = _read(p, [0, 200], ids, level, exact, 600)
+    b = _read(p, [0, 100, 200], ids, level, exact, 600)
+    assert np.abs(a[0]).max() > 0
+    for x, y in zip(a, b):
+        np.testing.assert_array_equal(x, y)
