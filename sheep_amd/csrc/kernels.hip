@@ -1492,11 +1492,9 @@ extern "C" __global__ __launch_bounds__(128) void sml_ropekv_d64(const sml_kattn
     extern "C" __global__ __launch_bounds__(256) void sml_attn_r##R(const sml_kattn a) { attn_body<R, 4, false>(a); } \
     extern "C" __global__ __launch_bounds__(256) void sml_attn_s64_r##R(const sml_kattn a) { attn_body<R, 4, false, 64>(a); } \
     extern "C" __global__ __launch_bounds__(512) void sml_attn8_r##R(const sml_kattn a) { attn_body<R, 8, false>(a); } \
-    extern "C" __global__ __launch_bounds__(512) void sml_attnc8_r##R(const sml_kattn a) { attn_body<R, 8, true>(a); } \
     extern "C" __global__ __launch_bounds__(512) void sml_attn8_s32_r##R(const sml_kattn a) { attn_body<R, 8, false, 32>(a); } \
     extern "C" __global__ __launch_bounds__(512) void sml_attn8_s64_r##R(const sml_kattn a) { attn_body<R, 8, false, 64>(a); } \
-    extern "C" __global__ __launch_bounds__(512) void sml_attnc8_s32_r##R(const sml_kattn a) { attn_body<R, 8, true, 32>(a); } \
-    extern "C" __global__ __launch_bounds__(512) void sml_attnc8_s64_r##R(const sml_kattn a) { attn_body<R, 8, true, 64>(a); }
+    extern "C" __global__ __launch_bounds__(512) void sml_attnc8_s32_r##R(const sml_kattn a) { attn_body<R, 8, true, 32>(a); }
 ATTN_KERNEL(1) ATTN_KERNEL(2) ATTN_KERNEL(3) ATTN_KERNEL(4) ATTN_KERNEL(5) ATTN_KERNEL(6) ATTN_KERNEL(7) ATTN_KERNEL(8)
 // head_dim 64 (suffix _d64): 64 positions per round of 8 waves, so splits of 64 or 128
 #define ATTN_KERNEL_D64(R) \

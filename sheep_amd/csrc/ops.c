@@ -928,7 +928,7 @@ void op_attention(hipStream_t st, const float * q, const float * k, const float 
         return;
     }
     // one sequence: the 8-wave kernel over attn_split positions, the split the
-    // exact prompt kernel (sml_attnc8) takes, so prompts read at level 1 equal
+    // level-1 prompt kernels (sml_pp_attn, sml_attnc8) take, so prompts read at level 1 equal
     // stepping bit for bit (SML_ATTN_WAVES applies to the batched step only)
     // splits past n_pos are not launched: the merge of the ones that are
     // equals the merge of all (empty splits add exact zeros)
@@ -1045,6 +1045,19 @@ void op_attention_batch(hipStream_t st, const float * qkv, int qkv_stride, uint1
                            2 * (size_t) 8 * rep * 128 * 4;
         snprintf(name, sizeof name, "sml_attnw_r%d", rep);
         hx_launch3(name, (unsigned) ns, (unsigned) n_kv, (unsigned) ((nseq + 15) / 16), 512, lds, st, &a);
+        hx_launch3("sml_attn_merge", (unsigned) n_head, 1, (unsigned) nseq, (unsigned) hd, 0, st, &a);
+        return;
+    }
+    if (causal && hd == 128 && ch >= 64) {
+        // level-1 prompts: a wave per entry over splits of 128 or 64 (a lane
+        // per position). It rotates q in place: qkv is the engine's scratch,
+        // read by nothing else. Splits of 32 (SML_ATTN_CHUNK only) and
+        // head_dim 64 stay on sml_attnc8.
+        const int rep = n_head / n_kv, rg = (rep + (rep + 3) / 4 - 1) / ((rep + 3) / 4);
+        hx_launch("sml_pp_ropeq", (unsigned) (((size_t) nseq * n_head * 16 + 255) / 256), 1, 256, 0, st, &a);
+        snprintf(name, sizeof name, "sml_pp_attn%s_r%d", ch == 64 ? "_s64" : "", rep);
+        hx_launch3(name, (unsigned) ns, (unsigned) n_kv, (unsigned) ((nseq + a.tpw - 1) / a.tpw), 512,
+                   (size_t) ch * (2 * 256 + 8 * 4 * rg), st, &a);
         hx_launch3("sml_attn_merge", (unsigned) n_head, 1, (unsigned) nseq, (unsigned) hd, 0, st, &a);
         return;
     }

@@ -973,3 +973,189 @@ extern "C" __global__ __launch_bounds__(256) void sml_pp_normq(const sml_knormq2
         }
     }
 }
+
+// ---------------------------------------------------------------- prompt attention in decoding's float order
+//
+// For prompts read at level 1, whose attention equals decoding's bit for bit.
+// Decoding spreads a position's 128 dims over 16 lanes and a split's positions
+// over 8 waves of 4 such rows; the values it computes are, per (entry, query
+// head, split): a score as 16 chains of 8 FMAs and their balanced tree; per
+// wave w (positions 4w..4w+3 of every 32) the max, the weights in base 2 and
+// their sum, each row's chain over the 32s and the tree over the 4 rows, for
+// the weights and for P V; then a chain over the waves. Here a wave takes a
+// whole entry and computes just these: the scores with a lane per position
+// (the chains and the tree in registers: no cross-lane adds), the 8 softmaxes
+// at once, 8 lanes each, P V with two dims a lane and the weights from LDS by
+// broadcast. K and V are staged once per 16 entries, straight to LDS (K's
+// 16-byte words swizzled by position); q comes rotated (sml_pp_ropeq, in
+// place) by scalar loads, and the FMAs take fp16 K and V as they are
+// (v_fma_mix). No barrier past the staging.
+// Bound by VALU issue (256 FMAs a position and head, 1.4 instructions each):
+// 512 rows at 509, 32 heads over 8: 226 us + 5.5, 620 with a 16-lane row per
+// position (cross-lane sums, q rotated by every row, two barriers an entry).
+extern "C" __global__ __launch_bounds__(256) void sml_pp_ropeq(const sml_kattn a) {
+    const int t = blockIdx.x * 256 + threadIdx.x;             // 4 dims of a row's first halves
+    const int per = a.n_head * 16, b = t / per;
+    if (b >= a.nseq) return;
+    const int h = (t - b * per) >> 4, d = 4 * (t & 15), pos = a.pos[b];
+    float * q = (float *) a.q + (size_t) b * a.qkv_stride + (size_t) h * 128 + d;
+    const float4 lo = *(const float4 *) q, hi = *(const float4 *) (q + 64);
+    const float4 c = *(const float4 *) (a.cos_t + (size_t) pos * 64 + d), s = *(const float4 *) (a.sin_t + (size_t) pos * 64 + d);
+    *(float4 *) q = make_float4(__builtin_fmaf(lo.x, c.x, -(hi.x * s.x)), __builtin_fmaf(lo.y, c.y, -(hi.y * s.y)),
+                                __builtin_fmaf(lo.z, c.z, -(hi.z * s.z)), __builtin_fmaf(lo.w, c.w, -(hi.w * s.w)));
+    *(float4 *) (q + 64) = make_float4(__builtin_fmaf(lo.x, s.x, hi.x * c.x), __builtin_fmaf(lo.y, s.y, hi.y * c.y),
+                                       __builtin_fmaf(lo.z, s.z, hi.z * c.z), __builtin_fmaf(lo.w, s.w, hi.w * c.w));
+}
+
+__device__ __forceinline__ float lane_val(float v, int l) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
+}
+
+template <int REP, int NL>
+__device__ void pa_body(const sml_kattn & a) {
+    constexpr int HD = 128, CH = 64 * NL, W = 8;
+    constexpr int NG = (REP + 3) / 4, RG = (REP + NG - 1) / NG;     // heads in groups of up to 4
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint8_t * lk = lds, * lv = lds + CH * 256;
+    float * lp = (float *) (lds + 2 * CH * 256) + wave * RG * CH;
+    const int kh = blockIdx.y, split = blockIdx.x, kvd = a.n_kv * HD, ns = a.nsplit;
+    const int b0 = blockIdx.z * a.tpw, b1 = min(b0 + a.tpw, a.nseq);
+    const int t0 = split * CH, tl = min(a.pos[b1 - 1] + 1, t0 + CH);
+    const float sl = a.inv * 1.44269504088896341f;
+    if (t0 < tl) {
+        const size_t at = (size_t) t0 * kvd + (size_t) kh * HD;
+        const uint16_t * kc = (a.kc_slots ? a.kc_slots[a.slot[b0]] + a.layer_off : a.kcache) + at;
+        const uint16_t * vc = (a.vc_slots ? a.vc_slots[a.slot[b0]] + a.layer_off : a.vcache) + at;
+        #pragma unroll
+        for (int i = 0; i < CH / (4 * W); i++) {
+            const int r0 = 4 * (W * i + wave), r = r0 + (lane >> 4), w = lane & 15;
+            const uint32_t row = (uint32_t) (t0 + r < tl ? r : 0) * (uint32_t) (kvd * 2);
+            copy_lds16(kc, row + 16u * (uint32_t) (w ^ (r & 15)), lk + r0 * 256);
+            copy_lds16(vc, row + 16u * (uint32_t) w, lv + r0 * 256);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    }
+    for (int b = b0 + wave; b < b1; b += W) {
+        const int T = a.pos[b] + 1;
+        float * blk = a.part + (size_t) b * a.n_head * ns * (HD + 2);
+        float2 * pml = (float2 *) (blk + (size_t) a.n_head * ns * HD) + (size_t) kh * REP * ns + split;
+        float * po = blk + ((size_t) kh * REP * ns + split) * HD + 2 * lane;
+        if (t0 >= T) {
+            if (lane < REP) pml[(size_t) lane * ns] = make_float2(-INFINITY, 0.0f);
+            continue;
+        }
+        const int n = min(T - t0, CH);
+        for (int g = 0; g < NG; g++) {
+            const __attribute__((address_space(4))) float * q[RG];
+            #pragma unroll
+            for (int j = 0; j < RG; j++)
+                q[j] = (const __attribute__((address_space(4))) float *) (a.q + (size_t) b * a.qkv_stride +
+                                                                          (size_t) (kh * REP + min(g * RG + j, REP - 1)) * HD);
+            // scores of positions lane, lane + 64: 16 chains of 8 and their tree
+            float sc[RG][NL], st[3][RG][NL];
+            #pragma unroll
+            for (int l = 0; l < 16; l++) {
+                v8h k[NL];
+                #pragma unroll
+                for (int u = 0; u < NL; u++) k[u] = *(const v8h *) (lk + (lane + 64 * u) * 256 + 16 * (l ^ (lane & 15)));
+                #pragma unroll
+                for (int j = 0; j < RG; j++)
+                    #pragma unroll
+                    for (int u = 0; u < NL; u++) {
+                        float p = 0.0f;
+                        #pragma unroll
+                        for (int e = 0; e < 8; e++) p = __builtin_fmaf(q[j][8 * l + e], (float) k[u][e], p);
+                        if (l & 1) p = st[0][j][u] + p;
+                        if ((l & 3) == 3) p = st[1][j][u] + p;
+                        if ((l & 7) == 7) p = st[2][j][u] + p;
+                        if (l == 15) p = sc[j][u] + p;
+                        if (!(l & 1)) st[0][j][u] = p;
+                        else if ((l & 3) == 1) st[1][j][u] = p;
+                        else if ((l & 7) == 3) st[2][j][u] = p;
+                        else sc[j][u] = p;
+                    }
+            }
+            // the softmax of each of decoding's 8 waves (wave w: positions 4w..4w+3
+            // of every 32), 8 lanes each here
+            float e[RG], lw[RG], L[RG], M[RG];
+            #pragma unroll
+            for (int j = 0; j < RG; j++) {
+                float m = -INFINITY;
+                #pragma unroll
+                for (int u = 0; u < NL; u++) {
+                    sc[j][u] = lane + 64 * u < n ? sc[j][u] * sl : -INFINITY;
+                    m = fmaxf(m, sc[j][u]);
+                }
+                m = fmaxf(m, dpp_f<0xB1>(m));
+                m = fmaxf(m, dpp_f<0x4E>(m));
+                m = fmaxf(m, __shfl_xor(m, 32));
+                const float mj = m == -INFINITY ? 0.0f : m;
+                float ls = 0.0f;
+                #pragma unroll
+                for (int u = 0; u < NL; u++) {
+                    const float p = __builtin_amdgcn_exp2f(sc[j][u] - mj), x = __shfl_xor(p, 32);
+                    lp[j * CH + 64 * u + lane] = p;
+                    ls += lane < 32 ? p : x;
+                    ls += lane < 32 ? x : p;
+                }
+                ls = ls + dpp_f<0xB1>(ls);
+                lw[j] = ls + dpp_f<0x4E>(ls);
+                float x = fmaxf(m, dpp_f<0x141>(m));
+                x = fmaxf(x, dpp_f<0x140>(x));
+                M[j] = fmaxf(x, swz16_f(x));                  // finite: wave 0 holds t0
+                e[j] = __builtin_amdgcn_exp2f(m - M[j]);
+                L[j] = 0.0f;
+            }
+            // P V for dims 2 lane, 2 lane + 1: each wave's four chains over the
+            // 32s, their sum, then the waves by their weights
+            float o[RG][2];
+            #pragma unroll
+            for (int j = 0; j < RG; j++) o[j][0] = o[j][1] = 0.0f;
+            #pragma unroll 1
+            for (int w = 0; w < W; w++) {
+                float acc[RG][4][2];
+                #pragma unroll
+                for (int j = 0; j < RG; j++)
+                    #pragma unroll
+                    for (int r = 0; r < 4; r++) acc[j][r][0] = acc[j][r][1] = 0.0f;
+                #pragma unroll
+                for (int i = 0; i < 2 * NL; i++) {
+                    v2h v[4];
+                    #pragma unroll
+                    for (int r = 0; r < 4; r++) v[r] = *(const v2h *) (lv + (32 * i + 4 * w + r) * 256 + 4 * lane);
+                    #pragma unroll
+                    for (int j = 0; j < RG; j++) {
+                        const float4 p = *(const float4 *) (lp + j * CH + 32 * i + 4 * w);
+                        const float pr[4] = {p.x, p.y, p.z, p.w};
+                        #pragma unroll
+                        for (int r = 0; r < 4; r++) {
+                            acc[j][r][0] = __builtin_fmaf(pr[r], (float) v[r][0], acc[j][r][0]);
+                            acc[j][r][1] = __builtin_fmaf(pr[r], (float) v[r][1], acc[j][r][1]);
+                        }
+                    }
+                }
+                #pragma unroll
+                for (int j = 0; j < RG; j++) {
+                    const float ew = lane_val(e[j], 4 * w);
+                    L[j] = __builtin_fmaf(ew, lane_val(lw[j], 4 * w), L[j]);
+                    #pragma unroll
+                    for (int d = 0; d < 2; d++)
+                        o[j][d] = __builtin_fmaf(ew, (acc[j][0][d] + acc[j][1][d]) + (acc[j][2][d] + acc[j][3][d]), o[j][d]);
+                }
+            }
+            #pragma unroll
+            for (int j = 0; j < RG; j++) {
+                const int h = g * RG + j;
+                if (h >= REP) continue;
+                *(float2 *) (po + (size_t) h * ns * HD) = make_float2(o[j][0], o[j][1]);
+                if (lane == 0) pml[(size_t) h * ns] = make_float2(M[j], L[j]);
+            }
+        }
+    }
+}
+#define PA_KERNEL(R)                                                                                                          \
+    extern "C" __global__ __launch_bounds__(512, 4) void sml_pp_attn_r##R(const sml_kattn a) { pa_body<R, 2>(a); }            \
+    extern "C" __global__ __launch_bounds__(512, 4) void sml_pp_attn_s64_r##R(const sml_kattn a) { pa_body<R, 1>(a); }
+PA_KERNEL(1) PA_KERNEL(2) PA_KERNEL(3) PA_KERNEL(4) PA_KERNEL(5) PA_KERNEL(6) PA_KERNEL(7) PA_KERNEL(8)
