@@ -616,7 +616,9 @@ PS_KERNEL(4, 4) PS_KERNEL(4, 8) PS_KERNEL(6, 4) PS_KERNEL(6, 8)
 //    rotates it) as two fp16 parts, q_hi = fp16(q) and q_lo = fp16(q - q_hi),
 //    so the scores carry q to ~2^-22; a lane then holds row l%16 at KV
 //    positions 4(l/16)..+3 of each 16-position tile;
-//  - the softmax in base 2 and fp32, masked past each entry's position;
+//  - the softmax in base 2 and fp32, masked past each entry's position, its
+//    first block as one over that block alone (a prompt of up to 64 positions
+//    sums in the order of the plain online form);
 //  - O += P V: A = P straight from the S^T layout (the MFMA's k slots
 //    8(l/16)..+7 hold KV rows 4(l/16)..+3 of two 16-position tiles), as fp16
 //    high and low parts like q (P rounded once to fp16, against a sum of the
@@ -628,7 +630,7 @@ PS_KERNEL(4, 4) PS_KERNEL(4, 8) PS_KERNEL(6, 4) PS_KERNEL(6, 8)
 // waves per SIMD (two workgroups per CU). What bounds it: matrix and vector
 // instructions of the same waves (64 MFMA of 16 clocks and ~220 others a
 // block), about half of the time each. 509 rows at 1531, 32 heads over 8:
-// 40 us, 124 with a wave per head, V transposed by 2-byte LDS writes (8 to
+// 42 us, 124 with a wave per head, V transposed by 2-byte LDS writes (8 to
 // a bank) and 2 waves per SIMD; 16 rows to a wave 42 against 45 for 32 (half
 // the LDS reads, half the waves).
 // One split: the output is written directly; several: partials of sml_attn's
@@ -745,27 +747,21 @@ __device__ void pf_body(const sml_kattn & a) {
         for (int u = 0; u < QT; u++) {
             // mask (the blocks that reach past a row's position) and the block's max for the lane's row
             const int lim = min(posq[u], t_end - 1) - t0 - 4 * g;
-            if (__any(lim < 48 + 3)) {
-                #pragma unroll
-                for (int j = 0; j < 4; j++)
-                    #pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        if (16 * j + r > lim) s[u][j][r] = -INFINITY;
-            }
             float mx = -INFINITY;
             #pragma unroll
             for (int j = 0; j < 4; j++)
                 #pragma unroll
-                for (int r = 0; r < 4; r++) mx = fmaxf(mx, s[u][j][r]);
-            mx *= sl;
-            // the base of the weights is 7 below the max (weights up to 128, so
-            // that fewer low parts fall below fp16's normal range) and moves
-            // only when the max has passed it by 15 (weights up to 2^15, within
-            // the range): most blocks need no reduction over the row's lanes
+                for (int r = 0; r < 4; r++) {
+                    s[u][j][r] = 16 * j + r <= lim ? s[u][j][r] * sl : -INFINITY;
+                    mx = fmaxf(mx, s[u][j][r]);
+                }
+            // the base of the weights is the first max and moves only when a
+            // later one passes it by 15 (weights up to 2^15, within fp16's
+            // range): most blocks need no reduction over the row's lanes
             if (__any(mx > m_run[u] + 15.0f)) {
                 mx = fmaxf(mx, __shfl_xor(mx, 16));
                 mx = fmaxf(mx, __shfl_xor(mx, 32));
-                const float m_new = mx > m_run[u] + 15.0f ? mx - 7.0f : m_run[u];
+                const float m_new = mx > m_run[u] + 15.0f ? mx : m_run[u];
                 // rescale O (its rows are 4g..4g+3)
                 const float alpha = __builtin_amdgcn_exp2f(m_run[u] - (m_new == -INFINITY ? 0.0f : m_new));
                 l_run[u] *= alpha;
@@ -784,8 +780,7 @@ __device__ void pf_body(const sml_kattn & a) {
             for (int j = 0; j < 4; j++)
                 #pragma unroll
                 for (int r = 0; r < 4; r += 2) {
-                    const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u][j][r], sl, -mu));
-                    const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u][j][r + 1], sl, -mu));
+                    const float p0 = __builtin_amdgcn_exp2f(s[u][j][r] - mu), p1 = __builtin_amdgcn_exp2f(s[u][j][r + 1] - mu);
                     ls += p0;
                     ls += p1;
                     const v2h ph = {(_Float16) p0, (_Float16) p1};
