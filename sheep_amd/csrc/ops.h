@@ -114,11 +114,11 @@ void op_attention(hipStream_t st, const float * q, const float * k, const float 
 // sequence's worth per b. causal: entries may be positions of one sequence
 // (prompt reading), so every k and v is rotated and written by one launch
 // before any entry attends; 1 keeps the decode kernel's arithmetic per entry
-// (bit-exact with stepping), 2 runs the wave-per-position kernel (faster,
-// its own fp32 order). The quantized out is per 32 values, or per 256 when
-// q256 (decode steps, causal 0, of an even head count only). n_pos bounds
-// every entry's position as in op_attention (the flash prompt form splits
-// the whole n_ctx range).
+// (bit-exact with stepping; at head_dim 128 it rotates q in place, so qkv is
+// the caller's scratch), 2 runs the MFMA flash form (faster, its own order).
+// The quantized out is per 32 values, or per 256 when q256 (decode steps,
+// causal 0, of an even head count only). n_pos bounds every entry's position
+// as in op_attention.
 // Exact mode's batched prompt rows (head_dim 128): every row's K/V written,
 // then each row's reference-order attention over positions 0..pos[b];
 // sc holds nrows * n_head * n_ctx floats of scores.
