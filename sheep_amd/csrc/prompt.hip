@@ -381,7 +381,7 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void copy_lds16(const void * base, uint32_t off, const void * dst) {
     const uint32_t at = (uint32_t) (uintptr_t) (const __attribute__((address_space(3))) void *) dst;
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :: "s"(__builtin_amdgcn_readfirstlane(at)), "v"(off), "s"(base) : "memory");
+                 :: "s"(__builtin_amdgcn_readfirstlane(at)), "v"(off), "s"(base) : "m0", "memory");
 }
 
 template <int NB, bool SW, int P>
