@@ -378,11 +378,14 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 // in flight before the next LDS read; the caller waits (vmcnt) and then meets
 // the other waves before any of the bytes is read. (Loads that the compiler
 // counts itself only ever wait longer for the copies it does not.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"             // m0 among the clobbers: it is what the statement sets
 __device__ __forceinline__ void copy_lds16(const void * base, uint32_t off, const void * dst) {
     const uint32_t at = (uint32_t) (uintptr_t) (const __attribute__((address_space(3))) void *) dst;
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                  :: "s"(__builtin_amdgcn_readfirstlane(at)), "v"(off), "s"(base) : "m0", "memory");
 }
+#pragma clang diagnostic pop
 
 template <int NB, bool SW, int P>
 __device__ void ps_body(const sml_kgemm & a) {
