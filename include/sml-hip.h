@@ -161,7 +161,8 @@ int sml_hip_gemm_swiglu(const sml_hip_mat * gate, const sml_hip_mat * up, const 
 // kernels, which are exact on such activations (the scale repeats in every
 // group). Above 16 rows (prompt reading) Q4 and Q6 run on the prompt GEMM:
 // tiles of 64 weight rows (SwiGLU: 32 of each matrix) x 64 or 128 positions,
-// the same integer superblock sums; other widths run in slices of 16 rows.
+// the same integer superblock sums; other widths, and codes q that are not
+// 16-byte aligned, run in slices of 16 rows.
 // replaces sml_matvec_batch_flat4_sb and sml_rlp_matvec
 // (sml/sml-kernel.c:1414-1435,1820-1840) as batch_group dispatches them in
 // the prompt and default multi-sequence regimes (sml/sml-run.c:2090-2150)
@@ -264,8 +265,8 @@ int sml_hip_attention(float * q, const float * k, const float * v, uint16_t * kc
 // floats); every row's k is rotated and its k and v written to the cache
 // before any row attends, then row b's heads attend over [0, pos0+b] into out
 // (n_rows x n_head*hd). The level-2 prompt's attention (the MFMA flash kernel,
-// its KV range split and merged as the grid needs; SML_ATTN_FLASH=0: a wave
-// per position), replacing the rope + f32_to_f16 + ms_attn of the reference's
+// its KV range split and merged as the grid needs; SML_ATTN_FLASH=0, or
+// caches that are not 16-byte aligned: a wave per position), replacing the rope + f32_to_f16 + ms_attn of the reference's
 // batched prompt body (sml/sml-run.c:2192-2210,2368-2378). hd must be 128,
 // n_kv at most 8; part holds n_rows*n_head*ceil(n_ctx/128)*(hd+2) floats.
 int sml_hip_attention_prompt(const float * qkv, int n_rows, int pos0, uint16_t * kcache, uint16_t * vcache,

@@ -14,6 +14,10 @@ static int env_int(const char * name, int dflt) {
     return e && *e ? atoi(e) : dflt;
 }
 
+// Whether the copies from memory straight into LDS (16 bytes a lane) may read
+// from here; the kernels' ordinary loads take any alignment of their type.
+static int al16(const void * p) { return ((uintptr_t) p & 15u) == 0; }
+
 static size_t al256(size_t x) { return (x + 255u) & ~(size_t) 255u; }
 
 // the split-K sums op_gemm left for the next normq (ops_defer_ksum)
@@ -1000,14 +1004,15 @@ void op_attention_batch(hipStream_t st, const float * qkv, int qkv_stride, uint1
     // head_dim 64 reads level-2 prompts with the level-1 kernel (the matrix-core
     // and wave-per-position prompt kernels are head_dim 128), at splits of
     // 128 as the level-2 partials are sized
-    const int c2_d64 = causal == 2 && hd == 64;
+    const int c2_d64 = causal >= 2 && hd == 64;
     if (c2_d64) causal = 1;
+    const int flash = causal == 2 && env_int("SML_ATTN_FLASH", 1);
     if (nseq < 1 || nseq > 65535) hx_failf("attention batch of %d", nseq);
     const int aw = env_int("SML_ATTN_WAVES", nseq >= 4 && !exact ? 4 : 8) == 4 ? 4 : 8;
     // the 8-wave kernels split as decoding does (attn_split); the 4-wave and
     // wave-per-position kernels run splits of 128
     const int bch = env_int("SML_ATTN_BCH", ATTN_CHUNK) == 64 && hd == 128 ? 64 : ATTN_CHUNK;
-    const int ch = causal == 2 || c2_d64 ? ATTN_CHUNK : causal == 0 && aw == 4 ? bch : attn_split(n_kv, n_ctx, hd);
+    const int ch = causal >= 2 || c2_d64 ? ATTN_CHUNK : causal == 0 && aw == 4 ? bch : attn_split(n_kv, n_ctx, hd);
     const int ns = (n_pos + ch - 1) / ch;             // splits past n_pos: not launched
     sml_kattn a;
     memset(&a, 0, sizeof a);
@@ -1033,12 +1038,12 @@ void op_attention_batch(hipStream_t st, const float * qkv, int qkv_stride, uint1
     a.nseq = nseq;
     a.tpw = causal ? env_int("SML_ATTN_TPW", 16) : 1;
     if (a.tpw < 1 || a.tpw > 16) a.tpw = 1;
-    if (causal == 2 && env_int("SML_ATTN_FLASH", 1)) {
+    if (flash) {
         if (q_out) hx_failf("flash prompt attention does not quantize its output");
         prompt_flash(st, &a, n_ctx, n_pos);
         return;
     }
-    if (causal == 2) {
+    if (causal >= 2) {
         // a wave per position over an LDS tile (16 positions per workgroup)
         const int rep = n_head / n_kv;
         const size_t lds = (size_t) ATTN_CHUNK * (128 + 8) * 2 + (size_t) ATTN_CHUNK * 128 * 2 +
@@ -1137,7 +1142,7 @@ int sml_hip_attention_prompt(const float * qkv, int n_rows, int pos0, uint16_t *
         hx_failf("prompt attention shape (heads %d/%d, head_dim %d) not supported", n_head, n_kv, hd);
     if (n_rows < 1 || n_rows > 65535 || pos0 < 0 || pos0 + n_rows > n_ctx)
         hx_failf("prompt attention over positions %d..%d of %d", pos0, pos0 + n_rows - 1, n_ctx);
-    if (hd == 128 && env_int("SML_ATTN_FLASH", 1)) {
+    if (al16(kcache) && al16(vcache) && hd == 128 && env_int("SML_ATTN_FLASH", 1)) {
         // one cache, consecutive positions: nothing to look up on the device
         sml_kattn a;
         memset(&a, 0, sizeof a);
@@ -1177,7 +1182,7 @@ int sml_hip_attention_prompt(const float * qkv, int n_rows, int pos0, uint16_t *
     }
     hx.jb = &jb;
     op_attention_batch(0, qkv, (n_head + 2 * n_kv) * hd, slots, slots + 1, slot, 0, cos_t, sin_t, slot + n_rows,
-                       n_rows, n_head, n_kv, hd, n_ctx, pos0 + n_rows, part, out, NULL, NULL, NULL, 2, 0, 0);
+                       n_rows, n_head, n_kv, hd, n_ctx, pos0 + n_rows, part, out, NULL, NULL, NULL, al16(kcache) && al16(vcache) ? 2 : 3, 0, 0);
     HX(hipDeviceSynchronize());
     hx.jb = outer;
     HX(hipFree(t));
@@ -1595,9 +1600,9 @@ void op_gemm(hipStream_t st, const sml_kmat * tab, const sml_kmat * hk, int ngro
     const int msmall = regime == GEMM_EXACT ? 32 : 16;
     if (!count && m_all > msmall) {
         // prompt-sized: Q4 and Q6 with per-256 activations on the prompt MFMA
-        // GEMM (ps_body); anything else in slices of msmall rows through the
-        // small-M kernels
-        if (per256 && hk && (nbits == 4 || nbits == 6) && cols % 256 == 0 && env_int("SML_PGEMM", 1)) {
+        // GEMM (ps_body), whose codes it copies into LDS; anything else in
+        // slices of msmall rows through the small-M kernels
+        if (per256 && hk && (nbits == 4 || nbits == 6) && cols % 256 == 0 && al16(q) && env_int("SML_PGEMM", 1)) {
             // 128 positions a workgroup where that alone fills the chip (the
             // weights' bytes are split for twice the positions: SwiGLU 2 x
             // 14336 x 4096 at 128 positions 61 us against 75, at 512 226

@@ -115,7 +115,8 @@ void op_attention(hipStream_t st, const float * q, const float * k, const float 
 // (prompt reading), so every k and v is rotated and written by one launch
 // before any entry attends; 1 keeps the decode kernel's arithmetic per entry
 // (bit-exact with stepping; at head_dim 128 it rotates q in place, so qkv is
-// the caller's scratch), 2 runs the MFMA flash form (faster, its own order).
+// the caller's scratch), 2 runs the MFMA flash form (faster, its own order;
+// the caches 16-byte aligned), 3 the wave-per-position form it replaces.
 // The quantized out is per 32 values, or per 256 when q256 (decode steps,
 // causal 0, of an even head count only). n_pos bounds every entry's position
 // as in op_attention.
