@@ -3,6 +3,10 @@
 // its own (prompt.hsaco), kernels named sml_pp_*.
 #include "dev.h"
 
+// four words of an array that is aligned as its elements only
+struct __attribute__((packed, aligned(4))) int4_a4 { int x, y, z, w; };
+struct __attribute__((packed, aligned(4))) float4_a4 { float x, y, z, w; };
+
 // The codes of chunk c as bytes: ca for group c&~1, cb for group c|1, each
 // over the chunk's 16 columns (0 .. 2^NB - 1).
 template <int NB>
@@ -868,7 +872,7 @@ extern "C" __global__ __launch_bounds__(256) void sml_pp_merge(const sml_kattn a
     if (idx >= a.nseq * a.n_head) return;
     const int b = idx / a.n_head, h = idx - b * a.n_head;
     const float * blk = a.part + (size_t) b * a.n_head * ns * 130;
-    const float4 * po = (const float4 *) (blk + (size_t) h * ns * 128) + l;
+    const float4_a4 * po = (const float4_a4 *) (blk + (size_t) h * ns * 128) + l;   // 8-byte aligned: odd splits of odd heads
     const float2 * pml = (const float2 *) (blk + (size_t) a.n_head * ns * 128) + (size_t) h * ns;
     float M = -INFINITY;
     for (int s = l; s < ns; s += 32) M = fmaxf(M, pml[s].x);
@@ -878,12 +882,12 @@ extern "C" __global__ __launch_bounds__(256) void sml_pp_merge(const sml_kattn a
     #pragma unroll 4
     for (int s = 0; s < ns; s++) {
         const float2 ml = pml[s];
-        const float4 v = po[s * 32];
+        const float4_a4 v = po[s * 32];
         const float e = __builtin_amdgcn_exp2f(ml.x - M);     // 0 for splits past the position
         L += e * ml.y;
         o.x += e * v.x; o.y += e * v.y; o.z += e * v.z; o.w += e * v.w;
     }
-    *((float4 *) (a.out + (size_t) idx * 128) + l) = make_float4(o.x / L, o.y / L, o.z / L, o.w / L);
+    *((float4_a4 *) (a.out + (size_t) idx * 128) + l) = {o.x / L, o.y / L, o.z / L, o.w / L};
 }
 
 // ---------------------------------------------------------------- normalization + quantization of many rows
@@ -895,8 +899,6 @@ extern "C" __global__ __launch_bounds__(256) void sml_pp_merge(const sml_kattn a
 // output gathers from there four columns a lane (a group of 32 is 8 lanes, a
 // superblock one wave).
 // 512 x 4096 with its norm: 9.1 us, 18.6 there (mean over a layer's four).
-struct __attribute__((packed, aligned(4))) int4_a4 { int x, y, z, w; };
-struct __attribute__((packed, aligned(4))) float4_a4 { float x, y, z, w; };
 extern "C" __global__ __launch_bounds__(256) void sml_pp_normq(const sml_knormq2 a) {
     extern __shared__ __align__(16) float y[];                // [n]
     __shared__ double red[4];

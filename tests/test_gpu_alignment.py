@@ -89,3 +89,36 @@ def test_caches_off_the_copy_alignment(off, heads, kv, n, pos0):
         assert np.abs(o - got[0][0]).max() <= tol
         np.testing.assert_array_equal(k, got[0][1])
         np.testing.assert_array_equal(v, got[0][2])
+
+
+@pytest.mark.parametrize("heads,kv,splits", [(3, 1, 3), (5, 5, 3), (7, 1, 4), (1, 1, 1)])
+def test_merge_of_odd_splits_into_any_output(monkeypatch, heads, kv, splits):
+    # an odd product of heads and splits puts every second row's partials, and
+    # the offset the output, on 8- and 4-byte boundaries
+    monkeypatch.setenv("SML_PF_NS", str(splits))
+    rng = np.random.default_rng(heads)
+    n, pos0, n_ctx = 43, 300, 512
+    ang = np.arange(n_ctx)[:, None] * (1e4 ** (-np.arange(64) / 64.0))
+    cos, sin = np.cos(ang).astype(np.float32), np.sin(ang).astype(np.float32)
+    qkv = rng.standard_normal((n, (heads + 2 * kv) * 128)).astype(np.float32)
+    kc, vc = (rng.standard_normal((n_ctx, kv * 128)).astype(np.float16) for _ in range(2))
+    d = [sa.DevBuf.of(x) for x in (qkv, kc.view(np.uint16), vc.view(np.uint16), cos, sin)]
+    got = []
+    for off in (0, 4):
+        part, out = sa.DevBuf(n * heads * 4 * 130 * 4), At(np.zeros((n, heads, 128), np.float32), off)
+        assert sa.lib().sml_hip_attention_prompt(d[0].ptr, n, pos0, d[1].ptr, d[2].ptr, d[3].ptr, d[4].ptr, heads, kv,
+                                                 128, n_ctx, part.ptr, out.ptr) == 0, sa.lib().sml_hip_last_error()
+        got.append(out.read())
+    np.testing.assert_array_equal(got[0], got[1])
+    K, V = (d[i].read(np.uint16).view(np.float16).reshape(n_ctx, kv, 128).astype(np.float64) for i in (1, 2))
+    p, rep = np.arange(pos0, pos0 + n), heads // kv
+    q = qkv[:, :heads * 128].reshape(n, heads, 128).astype(np.float64)
+    c, s = cos[p, None].astype(np.float64), sin[p, None].astype(np.float64)
+    q = np.concatenate([q[..., :64] * c - q[..., 64:] * s, q[..., :64] * s + q[..., 64:] * c], -1)
+    for h in range(heads):
+        x = q[:, h] @ K[:pos0 + n, h // rep].T / np.sqrt(128.0)
+        big = np.abs(x).max()
+        x[np.arange(pos0 + n)[None] > p[:, None]] = -np.inf
+        w = np.exp(x - x.max(1, keepdims=True))
+        want = (w / w.sum(1, keepdims=True)) @ V[:pos0 + n, h // rep]
+        assert np.abs(got[0][:, h] - want).max() <= (8.0 + big) * 2.0 ** -20 * np.abs(V).max(), h
