@@ -170,12 +170,12 @@ typedef struct {
     // sml_pp_flash (prompt flash form): KV positions per split (grid z), a
     // multiple of 64
     int fchunk;
-    // pos NULL (sml_ropekv, sml_pp_flash): entry b is at position pos0 + b
-    int pos0;
     // query-head subsets per kv head (the 8-wave kernels; 0 or 1: none):
     // grid y = n_kv * nsub, workgroup y takes kv head y / nsub and its query
     // heads (y % nsub) * REP .. +REP-1 (REP = n_head / n_kv / nsub)
     int nsub;
+    // pos NULL (sml_ropekv, sml_pp_flash): entry b is at position pos0 + b
+    int pos0;
 } sml_kattn;
 
 // Decode attention in the reference's float order (exact mode), two
