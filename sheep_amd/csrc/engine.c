@@ -1013,29 +1013,30 @@ static void rows_layer(int L, int ns, const int32_t * pos, const int32_t * slot,
     // that to its own launch)
     const int fuse_q = y->perm_o < 0 &&
                        (!sb || (!causal && G.H % 2 == 0 && G.hd == 128 && env_int("SML_MERGE_Q256", 1)));
-    // a level-1 or exact-mode prompt chunk attends in slices of rows whose
-    // partials (scores) fit the buffer; a slice's rows see the cache rows that
-    // it and the slices before it wrote
-    int sl = ns;
-    if (regime == GEMM_REF) sl = (int) (G.mpart_floats / ((size_t) G.H * (size_t) G.n_ctx));
-    else if (causal && regime == GEMM_EXACT) sl = op_attention_rows(G.H, G.KV, G.hd, G.n_ctx, G.pos_cap, G.mpart_floats);
-    if (sl < 1) hx_failf("attention partials of no row");
-    for (int r0 = 0; r0 < ns; r0 += sl) {
-        const int nr = ns - r0 < sl ? ns - r0 : sl;
-        const size_t ro = (size_t) r0 * hq;
-        int8_t * aq = fuse_q ? G.maq + ro : NULL;
-        float * as = fuse_q ? G.mas + ro / 32 : NULL;
-        int32_t * au = fuse_q ? G.masum + ro / 32 : NULL;
-        if (regime == GEMM_REF) {
-            // exact mode: one sequence (slot 0), the reference's order
-            if (!causal) hx_failf("exact mode batches prompts only");
-            op_attention_rows_exact(G.st, G.mqkv + (size_t) r0 * qkv, (int) qkv, G.kc + (size_t) L * G.n_ctx * kvd,
-                                    G.vc + (size_t) L * G.n_ctx * kvd, G.rc, G.rs, pos + r0, nr, G.H, G.KV, G.n_ctx,
-                                    G.pos_cap, G.mpart, G.matt + ro, aq, as, au);
-        } else {
+    if (regime == GEMM_REF) {
+        // exact mode: one sequence (slot 0), the reference's order. The scores
+        // of a chunk fit: the partials hold rrows * H * ceil(n_ctx / 128) *
+        // (hd + 2) floats.
+        if (!causal) hx_failf("exact mode batches prompts only");
+        if ((size_t) ns * (size_t) G.H * (size_t) G.n_ctx > G.mpart_floats) hx_failf("exact attention scores of %d rows", ns);
+        op_attention_rows_exact(G.st, G.mqkv, (int) qkv, G.kc + (size_t) L * G.n_ctx * kvd,
+                                G.vc + (size_t) L * G.n_ctx * kvd, G.rc, G.rs, pos, ns, G.H, G.KV, G.n_ctx,
+                                G.pos_cap, G.mpart, G.matt, fuse_q ? G.maq : NULL, fuse_q ? G.mas : NULL,
+                                fuse_q ? G.masum : NULL);
+    } else {
+        // a level-1 prompt chunk attends in slices of rows whose partials fit
+        // the buffer (which splits of 64 and 32 positions can exceed); a
+        // slice's rows see the cache rows that it and the slices before it wrote
+        int sl = ns;
+        if (causal && regime == GEMM_EXACT) sl = op_attention_rows(G.H, G.KV, G.hd, G.n_ctx, G.pos_cap, G.mpart_floats);
+        if (sl < 1) hx_failf("attention partials of no row");
+        for (int r0 = 0; r0 < ns; r0 += sl) {
+            const int nr = ns - r0 < sl ? ns - r0 : sl;
+            const size_t ro = (size_t) r0 * hq;
             op_attention_batch(G.st, G.mqkv + (size_t) r0 * qkv, (int) qkv, G.kc_tab, G.vc_tab, slot + r0,
                                (size_t) L * G.n_ctx * kvd, G.rc, G.rs, pos + r0, nr, G.H, G.KV, G.hd, G.n_ctx,
-                               G.pos_cap, G.mpart, G.matt + ro, aq, as, au,
+                               G.pos_cap, G.mpart, G.matt + ro, fuse_q ? G.maq + ro : NULL,
+                               fuse_q ? G.mas + ro / 32 : NULL, fuse_q ? G.masum + ro / 32 : NULL,
                                causal ? (regime == GEMM_EXACT ? 1 : 2) : 0, gemm_exact(regime, ns), sb);
         }
     }
@@ -1108,12 +1109,14 @@ static void launch_rows(int ns, const int32_t * tok, const int32_t * pos, const 
 //  - level 1: chunks of pb (512) positions (16 with MoE layers); every product
 //    is the GEMV's arithmetic and the attention the decode kernel's, so the
 //    cache, the residuals and the logits equal reading the prompt a token at
-//    a time, bit for bit.
+//    a time, bit for bit. (Where down reads h in order, stepping runs the
+//    h-quantizing SwiGLU GEMV, whose 16 lanes a row sum more than 16 groups in
+//    another order: equal to float rounding there.)
 //  - exact mode: chunks of pb through the reference-order GEMM and attention.
 //  - level 2: chunks of pb (512) positions in the reference's prompt regime
 //    (activations per 256 values, integer superblock sums: the CPU engine's
 //    default prompt arithmetic, sml/sml-run.c:1929-1945), Q4 products on the
-//    prompt MFMA GEMM, attention a wave per position.
+//    prompt MFMA GEMM, attention on the MFMA flash kernel.
 // A split model's prompt, layer by layer: each layer runs over every chunk
 // before the next starts, so a streamed layer crosses the host link once per
 // prompt instead of once per chunk. The residual rows of all n positions
