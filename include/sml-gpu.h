@@ -41,8 +41,11 @@ int sml_gpu_layers(int * of);
 
 // How a prompt is read: 0 a token at a time through the decode graph; 1 (the
 // default) batched in chunks of 512 positions (16 with MoE layers) with every
-// product in the GEMV's arithmetic, equal to stepping bit for bit; 2 batched
-// with the Q4 products on the matrix cores (MFMA), equal to float rounding.
+// product in the GEMV's arithmetic, equal to stepping bit for bit (to float
+// rounding where the down product reads h without a permutation and rows are
+// wider than 512: stepping then fuses h's quantization into a gate/up GEMV of
+// 16 lanes a row); 2 batched with the Q4 products on the matrix cores (MFMA),
+// equal to float rounding.
 // Exact mode (SML_EXACT=1) takes 2 as 1: chunks of 512 positions in the
 // reference CPU path's float order, equal to its stepping bit for bit.
 // replaces sml/sml-gpu.h:26 (sml/sml-gpu-fwd.c:2420-2423)
