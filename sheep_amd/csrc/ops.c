@@ -1053,9 +1053,16 @@ void op_attention_batch(hipStream_t st, const float * qkv, int qkv_stride, uint1
         hx_launch3("sml_attn_merge", (unsigned) n_head, 1, (unsigned) nseq, (unsigned) hd, 0, st, &a);
         return;
     }
-    if (causal && hd == 128 && ch >= 64) {
-        // level-1 prompts: a wave per entry over splits of 128 or 64 (a lane
-        // per position). It rotates q in place: qkv is the engine's scratch,
+    // few entries: the decode kernel itself, a workgroup per entry, kv head and
+    // split, while that is at most 3 workgroups a CU (32 heads over 8, whole
+    // prompts of two layers at level 1, us, against a wave per entry: 2 ids at 0
+    // 198 / 226, 16 at 500 511 / 559, 96 at 0 801 / 851; at 4 a CU 4 ids at 4000
+    // 261 / 257); SML_ATTN_FEW overrides the count of workgroups
+    const int few = causal && hd == 128 && ch >= 64 && (long) ns * n_kv * nseq <= env_int("SML_ATTN_FEW", 3 * hx.ncu);
+    if (few) a.tpw = 1;
+    if (causal && hd == 128 && ch >= 64 && !few) {
+        // else a wave per entry over splits of 128 or 64 (a lane per
+        // position). It rotates q in place: qkv is the engine's scratch,
         // read by nothing else. Splits of 32 (SML_ATTN_CHUNK only) and
         // head_dim 64 stay on sml_attnc8.
         const int rep = n_head / n_kv, rg = (rep + (rep + 3) / 4 - 1) / ((rep + 3) / 4);
@@ -1067,7 +1074,7 @@ void op_attention_batch(hipStream_t st, const float * qkv, int qkv_stride, uint1
         return;
     }
     const int nt = causal ? 512 : 64 * aw;
-    attn_name(name, sizeof name, a.tpw > 1 || causal ? "sml_attnc8" : aw == 4 ? "sml_attn" : "sml_attn8",
+    attn_name(name, sizeof name, a.tpw > 1 || (causal && !few) ? "sml_attnc8" : aw == 4 && !causal ? "sml_attn" : "sml_attn8",
               ch, hd, n_head / n_kv);
     // the 4-wave decode split with its inputs spread over the workgroup
     // (sml_attnb: the same values, half the registers); SML_ATTNB=0 keeps

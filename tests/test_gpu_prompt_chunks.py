@@ -39,7 +39,9 @@ def same(path, n, n_ctx, exact=False):
 # wider gate and up products over 16 lanes a row.
 @pytest.mark.parametrize("heads,n_ctx,n,perm", [(4, 128, 120, False), (4, 128, 65, False), (3, 512, 500, False),
                                                 (8, 128, 120, True), (3, 512, 500, True)])
-def test_level_1_slices_equal_stepping(tmp_path, heads, n_ctx, n, perm):
+@pytest.mark.parametrize("few", ["0", ""])                # a wave per entry; few entries: a workgroup each
+def test_level_1_slices_equal_stepping(tmp_path, monkeypatch, heads, n_ctx, n, perm, few):
+    monkeypatch.setenv("SML_ATTN_FEW", few)
     p = tmp_path / "m.ssf"
     sa.synth_model(p, n_layer=2, n_vocab=600, nbits=4, random_perm=perm, seed=n, n_embd=128 * heads, n_head=heads,
                    n_head_kv=1, n_ff=512)

@@ -3,7 +3,8 @@ float64 at the edges of its 128-row tiles, 64-position blocks and splits, over
 scores whose maximum climbs, falls or stays far below zero; and the
 row-a-workgroup normalization + quantization (sml_pp_normq, from 128 rows)
 against the form that fewer rows take, bit for bit; and the level-1 prompt's
-attention (sml_pp_attn) against decoding, bit for bit."""
+attention (sml_pp_attn, and the decode kernel for few entries) against
+decoding, bit for bit."""
 import numpy as np
 import pytest
 
@@ -97,13 +98,15 @@ def test_many_rows_quantize_as_few(tmp_path, monkeypatch, n_embd, n_head, kv, n_
         np.testing.assert_array_equal(x, y)
 
 
+@pytest.mark.parametrize("few", ["0", ""])                # a wave per entry; few entries: a workgroup each
 @pytest.mark.parametrize("chunk", [128, 64, 32])
 @pytest.mark.parametrize("heads,kv,n", [(1, 1, 18), (4, 2, 129), (3, 1, 140), (4, 1, 131), (5, 1, 80), (12, 2, 65),
                                         (7, 1, 64), (8, 1, 150)])
-def test_level_1_attention_equals_decoding(tmp_path, monkeypatch, heads, kv, n, chunk):
+def test_level_1_attention_equals_decoding(tmp_path, monkeypatch, heads, kv, n, chunk, few):
     # every head grouping, splits of each size, entries ending in, at and past
     # a split; two cuts, so that the second reads what the first wrote
     monkeypatch.setenv("SML_ATTN_CHUNK", str(chunk))
+    monkeypatch.setenv("SML_ATTN_FEW", few)
     p = tmp_path / "m.ssf"
     sa.synth_model(p, n_layer=2, n_vocab=600, nbits=4, random_perm=True, seed=heads, n_embd=128 * heads, n_head=heads,
                    n_head_kv=kv, n_ff=512)
