@@ -1574,14 +1574,45 @@ int gemm_exact(int regime, int m_all) {
 static int px_takes(int outputs, int m_all) {
     return m_all > 16 && (long) outputs * m_all >= env_int("SML_PX_OUT", 150000);
 }
-static void px_launch(hipStream_t st, const char * base, int nbits, int swiglu, sml_kgemm * a) {
+static void px_launch(hipStream_t st, int ref, int nbits, int swiglu, sml_kgemm * a) {
     const int rt = swiglu ? 32 : 64;
     const uint64_t tiles = (uint64_t) ((a->rows + rt - 1) / rt) * (uint64_t) ((a->m_all + 63) / 64);
     if (tiles > 0x7FFFFFFFull || (uint64_t) a->m_all * (uint64_t) a->cols >= (1ull << 32))
         hx_failf("prompt GEMM of %d rows x %d positions", a->rows, a->m_all);
     char name[32];
-    snprintf(name, sizeof name, "%s_q%d%s", base, nbits, swiglu ? "_s" : "");
+    // the reference order in at most a workgroup a CU: registers for all of it
+    snprintf(name, sizeof name, "sml_pp_%s_q%d%s%s", ref ? "xgemm" : "gemm", nbits, swiglu ? "_s" : "",
+             ref && tiles <= (uint64_t) hx.ncu ? "_f" : "");
     hx_launch(name, (unsigned) tiles, 1, 512, nbits == 8 ? PX_LDS + 8 * 68 * 4 : PX_LDS, st, a);
+}
+
+// Positions a workgroup of the prompt GEMM takes, in 16s. A superblock costs a
+// CU about alpha + beta x (the workgroups that the fullest CU takes), in
+// hundredths of a microsecond: more positions a workgroup share the splitting of
+// the weights' bytes, fewer fill the chip and leave less of the last tile empty.
+// Fitted to 10 shapes of 512 x 512 to 4096 x 14336, both products, 13 counts of
+// 17 to 512 positions each (rms 5 to 8%). Q4's larger tiles want a second
+// workgroup on the CU (4096 x 14336 SwiGLU at 256 positions: 110 us by 64, 131 by
+// 128). us at 32 / 64 / 96 / 128 positions a workgroup: 8960 x 1536 SwiGLU at 65
+// positions 21.1 / 22.5 / 19.5 / 22.6 and at 160 28 / 27.5 / 26 / 37, 14336 x 4096
+// SwiGLU at 512 341 / 204 / 214 / 174, 1536 x 1536 at 128 8.8 / 11.8 / 13 / 15.8.
+// SML_PS_P overrides.
+static int ps_positions(int nbits, uint64_t nrt, int m_all) {
+    static const struct { int alpha, beta; } cost[2][4] = { { { 30, 67 }, { 57, 77 }, { 60, 106 }, { 64, 127 } },
+                                                            { { 38, 89 }, { 44, 108 }, { 58, 123 }, { 81, 141 } } };
+    const int fp = env_int("SML_PS_P", 0);
+    if (fp == 2 || fp == 4 || fp == 6 || fp == 8) return fp;
+    int p = 2;
+    uint64_t best = 0;
+    for (int i = 0; i < 4; i++) {
+        const uint64_t np = 32u * (i + 1), tiles = nrt * (((uint64_t) m_all + np - 1) / np);
+        const uint64_t w = (tiles + (uint64_t) hx.ncu - 1) / (uint64_t) hx.ncu;
+        if (i && (uint64_t) m_all <= np / 2) break;              // half of the tile empty
+        if (nbits == 4 && i >= 2 && w < 2) continue;
+        const uint64_t c = (uint64_t) cost[nbits == 6][i].alpha + (uint64_t) cost[nbits == 6][i].beta * w;
+        if (!i || c < best) { best = c; p = 2 * (i + 1); }
+    }
+    return p;
 }
 
 void op_gemm(hipStream_t st, const sml_kmat * tab, const sml_kmat * hk, int ngroups, int swiglu, int nbits, int rows, int cols,
@@ -1600,7 +1631,7 @@ void op_gemm(hipStream_t st, const sml_kmat * tab, const sml_kmat * hk, int ngro
         a.q = q; a.scale = scale; a.sums = sums; a.y = y; a.bias = bias; a.resid = resid;
         a.m0[0] = hk[0];
         if (swiglu) a.m0[1] = hk[1];
-        px_launch(st, ref ? "sml_pp_xgemm" : "sml_pp_gemm", nbits, swiglu, &a);
+        px_launch(st, ref, nbits, swiglu, &a);
         return;
     }
     // the widest small-M launch: 32 rows in the exact regime (VALU), else 16

@@ -91,7 +91,7 @@ __device__ __forceinline__ void chunk_codes(const ChunkW<NB> & w, int c, v4u & c
 
 template <int V> struct Int { static constexpr int value = V; };
 
-template <int NB, bool SW, bool REF>
+template <int NB, bool SW, bool REF, bool FEW = false>
 __device__ void px_body(const sml_kgemm & a) {
     #pragma clang fp contract(off)
     typedef long v1l;
@@ -207,6 +207,7 @@ __device__ void px_body(const sml_kgemm & a) {
             #pragma unroll
             for (int r = 0; r < 4; r++) acc[j][t][r] = 0.0f;
     auto compute = [&](auto half) {                  // slots 4 half .. 4 half + 3
+        if (FEW && p0 + 16 * wp >= m_all) return;    // no position: the wave only stages
         #pragma unroll
         for (int gg = 0; gg < 4; gg++) {
             constexpr int H = decltype(half)::value;
@@ -329,6 +330,17 @@ PX_KERNELS(sml_pp_gemm_q, 8, false) PX_KERNELS(sml_pp_xgemm_q, 4, true) PX_KERNE
 
 // ---------------------------------------------------------------- prompt GEMM in the superblock regime
 //
+// The reference order in launches of at most a workgroup a CU, where a stage's
+// own latency is the time: registers for all of it (131 to 142, nothing
+// spilled), and waves without a position leave their SIMD to the others. Two
+// Qwen2.5-1.5B-shaped layers, exact mode, whole prompt of 2 / 32 / 64 ids (us):
+// Q8 423 / 451 / 480 -> 332 / 366 / 429, Q4 347 / 374 / 403 -> 315 / 345 / 387;
+// where a CU takes more workgroups the second one hides as much (Llama-3-8B
+// shape, Q4, 512 ids: 2907, 3048 so).
+#define PX_FEW(NB)                                                                                                           \
+    extern "C" __global__ __launch_bounds__(512, 2) void sml_pp_xgemm_q##NB##_f(const sml_kgemm a) { px_body<NB, false, true, true>(a); } \
+    extern "C" __global__ __launch_bounds__(512, 2) void sml_pp_xgemm_q##NB##_s_f(const sml_kgemm a) { px_body<NB, true, true, true>(a); }
+PX_FEW(4) PX_FEW(8)
 // Y[p][r] = W.a[p] for a chunk of prompt positions p (hundreds) and every row
 // r of a Q4 or Q6 matrix, in the reference's prompt regime (sml_quantize_act_sb
 // and flat4_sb_body, sml/sml-kernel.c:115-185,1142-1190): per superblock b of

@@ -49,3 +49,23 @@ def test_batched_prompt_equals_stepping(tmp_path, monkeypatch, shape, nb, n, exa
     for a, b in zip(logits(p, ids, 1, exact, 600), logits(p, ids, 0, exact, 600)):
         assert np.abs(b).max() > 0
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("nb", [4, 8])
+@pytest.mark.parametrize("n", [33, 512])
+def test_exact_prompt_past_a_workgroup_a_cu(tmp_path, nb, n):
+    # 512 positions: 288 and 320 tiles, more than the chip's compute units; 33: a workgroup with an empty quarter
+    p = tmp_path / "m.ssf"
+    sa.synth_model(p, n_layer=1, n_vocab=600, nbits=nb, random_perm=True, seed=nb, n_embd=2304, n_head=18, n_head_kv=6,
+                   n_ff=1280)
+    ids = np.random.default_rng(n).integers(0, 600, n).astype(np.int32)
+    d = sa.Decoder(p, n_ctx=600, exact=True)
+    try:
+        out = []
+        for level in (1, 0):
+            d.prompt_mode(level)
+            out.append(d.prefill(ids, 0, 600))
+    finally:
+        d.close()
+    assert np.abs(out[0]).max() > 0
+    np.testing.assert_array_equal(out[0], out[1])
