@@ -320,7 +320,10 @@ __device__ void px_body(const sml_kgemm & a) {
     }
 }
 
-// four waves a SIMD (two workgroups a CU): at most 128 registers
+// Four waves a SIMD (two workgroups a CU): at most 128 registers, and no
+// instance but sml_pp_xgemm_q4 fits: a lane's sums and chains, the pending tree
+// sums (32) and the next stage's loads spill 2 to 21 registers (Q4 4 and 6 of
+// the SwiGLU, Q7 and Q8 15 and 21) to scratch.
 #define PX_KERNELS(NAME, NB, REF)                                                                                    \
     extern "C" __global__ __launch_bounds__(512, 4) void NAME##NB(const sml_kgemm a) { px_body<NB, false, REF>(a); }   \
     extern "C" __global__ __launch_bounds__(512, 4) void NAME##NB##_s(const sml_kgemm a) { px_body<NB, true, REF>(a); }
