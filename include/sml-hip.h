@@ -160,7 +160,7 @@ int sml_hip_gemm_swiglu(const sml_hip_mat * gate, const sml_hip_mat * up, const 
 // applying the fp32 scales once per 256 columns; the rest runs the per-group
 // kernels, which are exact on such activations (the scale repeats in every
 // group). Above 16 rows (prompt reading) Q4 and Q6 run on the prompt GEMM:
-// tiles of 64 weight rows (SwiGLU: 32 of each matrix) x 64 or 128 positions,
+// tiles of 64 weight rows (SwiGLU: 32 of each matrix) x 32 to 128 positions,
 // the same integer superblock sums; other widths, and codes q that are not
 // 16-byte aligned, run in slices of 16 rows.
 // replaces sml_matvec_batch_flat4_sb and sml_rlp_matvec

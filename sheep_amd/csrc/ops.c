@@ -1641,16 +1641,9 @@ void op_gemm(hipStream_t st, const sml_kmat * tab, const sml_kmat * hk, int ngro
         // GEMM (ps_body), whose codes it copies into LDS; anything else in
         // slices of msmall rows through the small-M kernels
         if (per256 && hk && (nbits == 4 || nbits == 6) && cols % 256 == 0 && al16(q) && env_int("SML_PGEMM", 1)) {
-            // 128 positions a workgroup where that alone fills the chip (the
-            // weights' bytes are split for twice the positions: SwiGLU 2 x
-            // 14336 x 4096 at 128 positions 61 us against 75, at 512 226
-            // against 257), else 64 (4096 x 4096 at 256 30 against 41, at 512
-            // 48 against 53; 6144 x 4096 at 512 65 against 69)
             const int rt = swiglu ? 32 : 64;
             const uint64_t nrt = (uint64_t) ((rows + rt - 1) / rt);
-            int p = m_all > 64 && 4 * nrt * (uint64_t) ((m_all + 127) / 128) >= 7 * (uint64_t) hx.ncu ? 8 : 4;
-            const int fp = env_int("SML_PS_P", 0);
-            if (fp == 4 || fp == 8) p = fp;
+            const int p = ps_positions(nbits, nrt, m_all);
             const uint64_t tiles = nrt * (uint64_t) ((m_all + 16 * p - 1) / (16 * p));
             if (tiles > 0x7FFFFFFFull || (uint64_t) m_all * (uint64_t) cols >= (1ull << 32))
                 hx_failf("prompt GEMM of %d rows x %d positions", rows, m_all);

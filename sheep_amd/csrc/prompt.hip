@@ -330,9 +330,6 @@ __device__ void px_body(const sml_kgemm & a) {
 PX_KERNELS(sml_pp_gemm_q, 2, false) PX_KERNELS(sml_pp_gemm_q, 3, false) PX_KERNELS(sml_pp_gemm_q, 4, false)
 PX_KERNELS(sml_pp_gemm_q, 5, false) PX_KERNELS(sml_pp_gemm_q, 6, false) PX_KERNELS(sml_pp_gemm_q, 7, false)
 PX_KERNELS(sml_pp_gemm_q, 8, false) PX_KERNELS(sml_pp_xgemm_q, 4, true) PX_KERNELS(sml_pp_xgemm_q, 8, true)
-
-// ---------------------------------------------------------------- prompt GEMM in the superblock regime
-//
 // The reference order in launches of at most a workgroup a CU, where a stage's
 // own latency is the time: registers for all of it (131 to 142, nothing
 // spilled), and waves without a position leave their SIMD to the others. Two
@@ -344,6 +341,9 @@ PX_KERNELS(sml_pp_gemm_q, 8, false) PX_KERNELS(sml_pp_xgemm_q, 4, true) PX_KERNE
     extern "C" __global__ __launch_bounds__(512, 2) void sml_pp_xgemm_q##NB##_f(const sml_kgemm a) { px_body<NB, false, true, true>(a); } \
     extern "C" __global__ __launch_bounds__(512, 2) void sml_pp_xgemm_q##NB##_s_f(const sml_kgemm a) { px_body<NB, true, true, true>(a); }
 PX_FEW(4) PX_FEW(8)
+
+// ---------------------------------------------------------------- prompt GEMM in the superblock regime
+//
 // Y[p][r] = W.a[p] for a chunk of prompt positions p (hundreds) and every row
 // r of a Q4 or Q6 matrix, in the reference's prompt regime (sml_quantize_act_sb
 // and flat4_sb_body, sml/sml-kernel.c:115-185,1142-1190): per superblock b of
@@ -622,7 +622,8 @@ __device__ void ps_body(const sml_kgemm & a) {
 #define PS_KERNEL(NB, P)                                                                                              \
     extern "C" __global__ __launch_bounds__(256, 2) void sml_pp_sgemm_q##NB##_p##P(const sml_kgemm a) { ps_body<NB, false, P>(a); } \
     extern "C" __global__ __launch_bounds__(256, 2) void sml_pp_sgemm_q##NB##_s_p##P(const sml_kgemm a) { ps_body<NB, true, P>(a); }
-PS_KERNEL(4, 4) PS_KERNEL(4, 8) PS_KERNEL(6, 4) PS_KERNEL(6, 8)
+PS_KERNEL(4, 2) PS_KERNEL(4, 4) PS_KERNEL(4, 6) PS_KERNEL(4, 8)
+PS_KERNEL(6, 2) PS_KERNEL(6, 4) PS_KERNEL(6, 6) PS_KERNEL(6, 8)
 
 // ---------------------------------------------------------------- prompt attention on MFMA (flash form)
 //

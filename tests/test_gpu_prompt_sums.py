@@ -57,14 +57,15 @@ def test_sums_at_the_edges(monkeypatch, nb, rows, cols, npos, extreme):
     up, uw = matrix(rng, rows, cols, nb, extreme)
     (q, s, u), a = acts(rng, npos, cols, extreme)
     got = {}
-    for p in ("4", "8"):                      # 64 and 128 positions a workgroup
+    for p in ("2", "4", "6", "8"):            # 32 to 128 positions a workgroup
         monkeypatch.setenv("SML_PS_P", p)
         y, h = sa.DevBuf(npos * rows * 4), sa.DevBuf(npos * rows * 4)
         sa.gemm(gate, q, s, u, npos, y, per256=True)
         sa.gemm_swiglu(gate, up, q, s, u, npos, h, per256=True)
         got[p] = [b.read(np.float32).reshape(npos, rows) for b in (y, h)]
-    for x, z in zip(got["4"], got["8"]):
-        np.testing.assert_array_equal(x, z)
+    for p in ("2", "6", "8"):
+        for x, z in zip(got["4"], got[p]):
+            np.testing.assert_array_equal(x, z)
     # each superblock's two products and sums round once: cols / 256 * 4
     # roundings of 2^-24, of terms up to the sum of the magnitudes
     want = a @ gw.T
