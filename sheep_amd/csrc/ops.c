@@ -1567,12 +1567,17 @@ int gemm_exact(int regime, int m_all) {
 #define PX_LDS (2 * 8 * 2 * (64 * 16 + 16) + 64 * 80 + 2 * 8 * 68 * 4)
 // Whether the exact regime takes it over the VALU GEMM. A launch costs a
 // tile's latency however few positions it holds (2.1 us per 256 columns), the
-// VALU GEMM about a fixed time per output, so the line is one on the outputs:
-// 4096 x 4096 crosses near 30 positions (32: 37 us against 42; 17: 37 against
-// 25), 4096 x 14336 near 40 (32: 114 against 92; 64: 117 against 182), 2 x
-// 14336 x 4096 below 17 (60 against 80 at 16). SML_PX_OUT overrides (tests).
+// VALU GEMM a launch for every 32 positions and, in it, about a fixed time per
+// output. So above 32 positions it always does, and up to 32 from 150000
+// outputs: whole prompts of four layers, us, matrix cores / VALU: 4096 and 14336
+// columns 17 ids 1230 / 1093 (880 with the line), 32 1248 / 1690 (1152), 40 1276 /
+// 2102; 1536 and 8960 17 ids 794 / 634 (570), 32 801 / 930 (765), 40 806 / 1207,
+// 64 823 / 1725; 512 and 1024 32 ids 366 / 490, 64 362 / 798. SML_PX_OUT sets
+// the line for every count above 16 (tests).
 static int px_takes(int outputs, int m_all) {
-    return m_all > 16 && (long) outputs * m_all >= env_int("SML_PX_OUT", 150000);
+    const int line = env_int("SML_PX_OUT", -1);
+    if (line >= 0) return m_all > 16 && (long) outputs * m_all >= line;
+    return m_all > 32 || (m_all > 16 && (long) outputs * m_all >= 150000);
 }
 static void px_launch(hipStream_t st, int ref, int nbits, int swiglu, sml_kgemm * a) {
     const int rt = swiglu ? 32 : 64;
