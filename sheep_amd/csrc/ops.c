@@ -549,10 +549,17 @@ void op_normq_rows(hipStream_t st, float * x, const float * resid, const float *
         memset(&b, 0, sizeof b);
         b.x = x; b.norm_w = w; b.eps = eps; b.n = n; b.nout = nout; b.per256 = per256; b.exact = g_exact;
         for (int i = 0; i < nout; i++) { b.perm[i] = perm[i]; b.q[i] = q[i]; b.scale[i] = scale[i]; b.sums[i] = sums[i]; }
-        // a workgroup a row from 128 rows: at n = 4096 (mean over a layer's
-        // calls, us) 32 rows 6.7 against 5.2 for a workgroup per 256 values,
-        // 64 6.6 / 5.4, 128 6.8 / 7.3, 256 7.5 / 11.3, 512 9.1 / 18.6
-        if (rows >= 128) hx_launch("sml_pp_normq", (unsigned) rows, 1, 256, (size_t) n * 4, st, &b);
+        // a workgroup a row from 192 rows where columns are gathered through a
+        // permutation, 256 where they are read in order (the old form then
+        // reads nothing twice): whole prompts of four layers, level 2, us, a
+        // workgroup a row / per 256 values: 4096 and 14336 columns, permuted,
+        // 128 ids 1016 / 1001, 192 1276 / 1312, 512 1982 / 2212, in order 128
+        // 978 / 968, 256 1307 / 1352; 1536 and 8960, permuted, 128 543 / 525,
+        // 192 572 / 573, 256 603 / 626, in order 128 521 / 496, 256 586 / 586,
+        // 512 845 / 888
+        int np = 0;
+        for (int i = 0; i < nout; i++) np += perm[i] != NULL;
+        if (rows >= (np ? 192 : 256)) hx_launch("sml_pp_normq", (unsigned) rows, 1, 256, (size_t) n * 4, st, &b);
         else hx_launch("sml_normq2", (unsigned) ((n + 255) / 256), (unsigned) rows, 256, 0, st, &b);
         return;
     }

@@ -1,7 +1,7 @@
 """Prompt rows: the matrix-core attention (sml_pp_flash, sml_pp_merge) against
 float64 at the edges of its 128-row tiles, 64-position blocks and splits, over
 scores whose maximum climbs, falls or stays far below zero; and the
-row-a-workgroup normalization + quantization (sml_pp_normq, from 128 rows)
+row-a-workgroup normalization + quantization (sml_pp_normq, many rows)
 against the form that fewer rows take, bit for bit; and the level-1 prompt's
 attention (sml_pp_attn, and the decode kernel for few entries) against
 decoding, bit for bit."""
@@ -80,19 +80,20 @@ def _read(path, cuts, ids, level, exact, vocab):
 
 @pytest.mark.parametrize("level,exact", [(1, False), (1, True), (2, False)])
 @pytest.mark.parametrize("n_embd,n_head,kv,n_ff", [(384, 3, 1, 1280), (1024, 8, 1, 1152), (2304, 18, 6, 2304)])
-def test_many_rows_quantize_as_few(tmp_path, monkeypatch, n_embd, n_head, kv, n_ff, level, exact):
-    # 128 rows and more in one read against reads of 100: the products and the
-    # wave-per-position attention do not depend on the cut
+@pytest.mark.parametrize("perm,n", [(True, 200), (False, 300)])
+def test_many_rows_quantize_as_few(tmp_path, monkeypatch, n_embd, n_head, kv, n_ff, level, exact, perm, n):
+    # 192 (permuted) and 256 rows and more in one read against reads of half:
+    # the products and the wave-per-position attention do not depend on the cut
     if exact and (n_ff % 256 or n_embd % 256):
         pytest.skip("exact mode batches 256-aligned products")
     monkeypatch.setenv("SML_ATTN_FLASH", "0")
     monkeypatch.setenv("SML_PX_OUT", "0")
     p = tmp_path / "m.ssf"
-    sa.synth_model(p, n_layer=2, n_vocab=600, nbits=4, random_perm=True, seed=n_embd, n_embd=n_embd, n_head=n_head,
+    sa.synth_model(p, n_layer=2, n_vocab=600, nbits=4, random_perm=perm, seed=n_embd, n_embd=n_embd, n_head=n_head,
                    n_head_kv=kv, n_ff=n_ff)
-    ids = np.random.default_rng(n_ff).integers(0, 600, 200).astype(np.int32)
-    a = _read(p, [0, 200], ids, level, exact, 600)
-    b = _read(p, [0, 100, 200], ids, level, exact, 600)
+    ids = np.random.default_rng(n_ff).integers(0, 600, n).astype(np.int32)
+    a = _read(p, [0, n], ids, level, exact, 600)
+    b = _read(p, [0, n // 2, n], ids, level, exact, 600)
     assert np.abs(a[0]).max() > 0
     for x, y in zip(a, b):
         np.testing.assert_array_equal(x, y)
