@@ -2,11 +2,12 @@
 where they can go wrong: values and steps at and past the range that the
 reciprocal form admits (both sides of 2^+-60, subnormals, infinities, NaN),
 exact ties, every code width, weights and partial codes; equal and NaN column
-keys, rows past the LDS and a perm that is only 4-byte aligned. All bit for
-bit (the quotients are the correctly rounded ones)."""
+keys, rows past the LDS and weights and orders that are only 4-byte aligned. All
+bit for bit (the quotients are the correctly rounded ones)."""
 import numpy as np
 import pytest
 
+import sheep_amd as sa
 from oracle import bind as ob
 from sheep_amd import ingest
 
@@ -91,3 +92,35 @@ def test_column_order(cols):
     h = res.host()
     for k in ("perm", "sd", "sq", "md", "mq", "codes"):
         assert np.array_equal(h[k], ref[k]), k
+
+
+@pytest.mark.parametrize("given", [False, True])
+@pytest.mark.parametrize("cols", [768, 41216])
+def test_column_order_of_unaligned_arrays(cols, given):
+    # the weights, the order asked for and the order written 4 bytes past a
+    # 16-byte boundary: what the aligned call gives, in and past the LDS
+    rng = np.random.default_rng(cols)
+    rows, nbits = 3, 4
+    w = (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32)
+    order = rng.permutation(cols).astype(np.int32) if given else None
+    got = []
+    for off in (0, 4):
+        wd = sa.DevBuf(w.nbytes + 16)
+        assert sa.lib().sml_hip_h2d(wd.ptr + off, w.ctypes.data, w.nbytes) == 0
+        od = None
+        if given:
+            od = sa.DevBuf(order.nbytes + 16)
+            assert sa.lib().sml_hip_h2d(od.ptr + off, order.ctypes.data, order.nbytes) == 0
+        r = ingest.Requantized(rows, cols, nbits, True)
+        perm = sa.DevBuf(cols * 4 + 16)
+        assert ingest._lib().sml_hip_requant(wd.ptr + off, rows, cols, nbits, od.ptr + off if given else None, None, 2,
+                                             r._pl(), r.sd.ptr, r.sq.ptr, r.md.ptr, r.mq.ptr, perm.ptr + off,
+                                             r.codes.ptr) == 0, sa.lib().sml_hip_last_error()
+        h = r.host()
+        h["perm"] = perm.read(np.uint8)[off:off + cols * 4].copy().view(np.int32)
+        got.append(h)
+    if given:
+        assert np.array_equal(got[1]["perm"], order)
+    for k in ("perm", "sd", "sq", "md", "mq", "codes"):
+        assert np.array_equal(got[0][k], got[1][k]), k
+    assert all(np.array_equal(a, b) for a, b in zip(got[0]["planes"], got[1]["planes"]))
