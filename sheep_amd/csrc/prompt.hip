@@ -666,7 +666,7 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 #define PF_STAGE (2 * PF_KB * 256)                      // its K rows, then its V rows
 
 __device__ void pf_body(const sml_kattn & a) {
-    constexpr int W = 8, QT = 1, HD = 128, RW = 16 * QT;               // rows (query, head) of a wave
+    constexpr int W = 8, HD = 128, RW = 16;                            // rows (query, head) of a wave
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, i16 = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -682,14 +682,13 @@ __device__ void pf_body(const sml_kattn & a) {
     const uint16_t * kc = (a.kc_slots ? a.kc_slots[a.slot[entry(rb)]] : a.kcache) + sl_off + (size_t) kh * HD;
     const uint16_t * vc = (a.vc_slots ? a.vc_slots[a.slot[entry(rb)]] : a.vcache) + sl_off + (size_t) kh * HD;
 
-    // the rotated q of each tile's row i16, dims 32c + 8g + e, as fp16 B operands (hi, lo)
+    // the rotated q of row i16, dims 32c + 8g + e, as fp16 B operands (hi, lo)
     const float sl = a.inv * 1.44269504088896341f;
-    v8h qb[QT][4], ql[QT][4];
-    int posq[QT];
-    #pragma unroll
-    for (int u = 0; u < QT; u++) {
-        const int row = min(rw + 16 * u + i16, nrow - 1), b = row / rep, h = kh * rep + (row - b * rep);
-        posq[u] = at(b);
+    v8h qb[4], ql[4];
+    int posq;
+    {
+        const int row = min(rw + i16, nrow - 1), b = row / rep, h = kh * rep + (row - b * rep);
+        posq = at(b);
         const float * qp = a.q + (size_t) b * a.qkv_stride + (size_t) h * HD + 8 * g;
         float x[4][8];
         #pragma unroll
@@ -701,8 +700,8 @@ __device__ void pf_body(const sml_kattn & a) {
             float cs[8], sn[8];
             #pragma unroll
             for (int e = 0; e < 8; e += 4) {
-                *(float4 *) &cs[e] = *(const float4 *) (a.cos_t + (size_t) posq[u] * half + 32 * c + 8 * g + e);
-                *(float4 *) &sn[e] = *(const float4 *) (a.sin_t + (size_t) posq[u] * half + 32 * c + 8 * g + e);
+                *(float4 *) &cs[e] = *(const float4 *) (a.cos_t + (size_t) posq * half + 32 * c + 8 * g + e);
+                *(float4 *) &sn[e] = *(const float4 *) (a.sin_t + (size_t) posq * half + 32 * c + 8 * g + e);
             }
             #pragma unroll
             for (int e = 0; e < 8; e++) {
@@ -715,20 +714,15 @@ __device__ void pf_body(const sml_kattn & a) {
         for (int c = 0; c < 4; c++)
             #pragma unroll
             for (int e = 0; e < 8; e++) {
-                qb[u][c][e] = (_Float16) x[c][e];
-                ql[u][c][e] = (_Float16) (x[c][e] - (float) qb[u][c][e]);
+                qb[c][e] = (_Float16) x[c][e];
+                ql[c][e] = (_Float16) (x[c][e] - (float) qb[c][e]);
             }
     }
-    float m_run[QT];                                    // of row i16 of each tile (the same in its 4 lanes)
-    float l_run[QT];                                    // the lane's positions' share of its sum
-    v4f o[QT][8];
+    float m_run = -INFINITY;                            // of row i16 (the same in its 4 lanes)
+    float l_run = 0.0f;                                 // the lane's positions' share of its sum
+    v4f o[8];
     #pragma unroll
-    for (int u = 0; u < QT; u++) {
-        m_run[u] = -INFINITY;
-        l_run[u] = 0.0f;
-        #pragma unroll
-        for (int dt = 0; dt < 8; dt++) o[u][dt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-    }
+    for (int dt = 0; dt < 8; dt++) o[dt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 
     // a block's rows into LDS: 16-byte word w of row r at place w ^ 2(r & 7);
     // rows past the range repeat its first
@@ -750,74 +744,67 @@ __device__ void pf_body(const sml_kattn & a) {
     auto compute = [&](int buf, int t0) {
         const uint8_t * st = lds + buf * PF_STAGE;
         // S^T: 4 tiles of 16 positions x 16 rows
-        v4f s[QT][4];
+        v4f s[4];
         #pragma unroll
         for (int j = 0; j < 4; j++) {
-            #pragma unroll
-            for (int u = 0; u < QT; u++) s[u][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            s[j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
             #pragma unroll
             for (int c = 0; c < 4; c++) {
                 const v8h ka = *(const v8h *) (st + 16 * j * 256 + krow + 16 * ((4 * c + g) ^ kx));
-                #pragma unroll
-                for (int u = 0; u < QT; u++) {
-                    s[u][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qb[u][c], s[u][j], 0, 0, 0);
-                    s[u][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, ql[u][c], s[u][j], 0, 0, 0);
-                }
+                s[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qb[c], s[j], 0, 0, 0);
+                s[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, ql[c], s[j], 0, 0, 0);
             }
         }
-        v8h pa[QT][2], pl[QT][2];
+        v8h pa[2], pl[2];
+        // mask (the blocks that reach past a row's position) and the block's max for the lane's row
+        const int lim = min(posq, t_end - 1) - t0 - 4 * g;
+        float mx = -INFINITY;
         #pragma unroll
-        for (int u = 0; u < QT; u++) {
-            // mask (the blocks that reach past a row's position) and the block's max for the lane's row
-            const int lim = min(posq[u], t_end - 1) - t0 - 4 * g;
-            float mx = -INFINITY;
+        for (int j = 0; j < 4; j++)
             #pragma unroll
-            for (int j = 0; j < 4; j++)
-                #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    s[u][j][r] = 16 * j + r <= lim ? s[u][j][r] * sl : -INFINITY;
-                    mx = fmaxf(mx, s[u][j][r]);
-                }
-            // the base of the weights is the first max and moves only when a
-            // later one passes it by 15 (weights up to 2^15, within fp16's
-            // range): most blocks need no reduction over the row's lanes
-            if (__any(mx > m_run[u] + 15.0f)) {
-                mx = fmaxf(mx, __shfl_xor(mx, 16));
-                mx = fmaxf(mx, __shfl_xor(mx, 32));
-                const float m_new = mx > m_run[u] + 15.0f ? mx : m_run[u];
-                // rescale O (its rows are 4g..4g+3)
-                const float alpha = __builtin_amdgcn_exp2f(m_run[u] - (m_new == -INFINITY ? 0.0f : m_new));
-                l_run[u] *= alpha;
-                float al[4];
-                #pragma unroll
-                for (int r = 0; r < 4; r++) al[r] = __shfl(alpha, 4 * g + r);
-                #pragma unroll
-                for (int dt = 0; dt < 8; dt++)
-                    #pragma unroll
-                    for (int r = 0; r < 4; r++) o[u][dt][r] *= al[r];
-                m_run[u] = m_new;
+            for (int r = 0; r < 4; r++) {
+                s[j][r] = 16 * j + r <= lim ? s[j][r] * sl : -INFINITY;
+                mx = fmaxf(mx, s[j][r]);
             }
-            const float mu = m_run[u] == -INFINITY ? 0.0f : m_run[u];   // no position yet: keep zeros
-            float ls = 0.0f;
+        // the base of the weights is the first max and moves only when a
+        // later one passes it by 15 (weights up to 2^15, within fp16's
+        // range): most blocks need no reduction over the row's lanes
+        if (__any(mx > m_run + 15.0f)) {
+            mx = fmaxf(mx, __shfl_xor(mx, 16));
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            const float m_new = mx > m_run + 15.0f ? mx : m_run;
+            // rescale O (its rows are 4g..4g+3)
+            const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new == -INFINITY ? 0.0f : m_new));
+            l_run *= alpha;
+            float al[4];
             #pragma unroll
-            for (int j = 0; j < 4; j++)
+            for (int r = 0; r < 4; r++) al[r] = __shfl(alpha, 4 * g + r);
+            #pragma unroll
+            for (int dt = 0; dt < 8; dt++)
                 #pragma unroll
-                for (int r = 0; r < 4; r += 2) {
-                    const float p0 = __builtin_amdgcn_exp2f(s[u][j][r] - mu), p1 = __builtin_amdgcn_exp2f(s[u][j][r + 1] - mu);
-                    ls += p0;
-                    ls += p1;
-                    const v2h ph = {(_Float16) p0, (_Float16) p1};
-                    float r0, r1;                             // p - hi, exact
-                    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r0) : "v"(ph), "v"(p0));
-                    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r1) : "v"(ph), "v"(p1));
-                    const v2h pr = {(_Float16) r0, (_Float16) r1};
-                    pa[u][j >> 1][4 * (j & 1) + r] = ph[0];
-                    pa[u][j >> 1][4 * (j & 1) + r + 1] = ph[1];
-                    pl[u][j >> 1][4 * (j & 1) + r] = pr[0];
-                    pl[u][j >> 1][4 * (j & 1) + r + 1] = pr[1];
-                }
-            l_run[u] += ls;
+                for (int r = 0; r < 4; r++) o[dt][r] *= al[r];
+            m_run = m_new;
         }
+        const float mu = m_run == -INFINITY ? 0.0f : m_run;   // no position yet: keep zeros
+        float ls = 0.0f;
+        #pragma unroll
+        for (int j = 0; j < 4; j++)
+            #pragma unroll
+            for (int r = 0; r < 4; r += 2) {
+                const float p0 = __builtin_amdgcn_exp2f(s[j][r] - mu), p1 = __builtin_amdgcn_exp2f(s[j][r + 1] - mu);
+                ls += p0;
+                ls += p1;
+                const v2h ph = {(_Float16) p0, (_Float16) p1};
+                float r0, r1;                             // p - hi, exact
+                asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r0) : "v"(ph), "v"(p0));
+                asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r1) : "v"(ph), "v"(p1));
+                const v2h pr = {(_Float16) r0, (_Float16) r1};
+                pa[j >> 1][4 * (j & 1) + r] = ph[0];
+                pa[j >> 1][4 * (j & 1) + r + 1] = ph[1];
+                pl[j >> 1][4 * (j & 1) + r] = pr[0];
+                pl[j >> 1][4 * (j & 1) + r + 1] = pr[1];
+            }
+        l_run += ls;
         // O += P V: per 32 positions k, slots 8g..8g+3 are rows 4g..4g+3 of
         // tile 2k, 8g+4..8g+7 those of tile 2k+1
         #pragma unroll
@@ -829,11 +816,8 @@ __device__ void pf_body(const sml_kattn & a) {
                 const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lv4s *) (vr + 32 * k * 256));
                 const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lv4s *) (vr + (32 * k + 16) * 256));
                 const v8h w = __builtin_bit_cast(v8h, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-                #pragma unroll
-                for (int u = 0; u < QT; u++) {
-                    o[u][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[u][k], w, o[u][dt], 0, 0, 0);
-                    o[u][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl[u][k], w, o[u][dt], 0, 0, 0);
-                }
+                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[k], w, o[dt], 0, 0, 0);
+                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl[k], w, o[dt], 0, 0, 0);
             }
         }
     };
@@ -851,28 +835,25 @@ __device__ void pf_body(const sml_kattn & a) {
 
     // the lane's rows: 4g..4g+3 of each tile, dims 16dt + i16
     const bool one = gridDim.z == 1;
+    l_run += __shfl_xor(l_run, 16);
+    l_run += __shfl_xor(l_run, 32);
     #pragma unroll
-    for (int u = 0; u < QT; u++) {
-        l_run[u] += __shfl_xor(l_run[u], 16);
-        l_run[u] += __shfl_xor(l_run[u], 32);
-        #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const float lq = __shfl(l_run[u], 4 * g + r), mq = __shfl(m_run[u], 4 * g + r);
-            const int row = rw + 16 * u + 4 * g + r;
-            if (row >= nrow) continue;
-            const int b = row / rep, h = kh * rep + (row - b * rep);
-            if (one) {
-                float * out = a.out + (size_t) b * a.n_head * HD + (size_t) h * HD;
-                #pragma unroll
-                for (int dt = 0; dt < 8; dt++) out[16 * dt + i16] = o[u][dt][r] / lq;
-            } else {
-                float * blk = a.part + (size_t) b * a.n_head * a.nsplit * (HD + 2);
-                float * po = blk + ((size_t) h * a.nsplit + blockIdx.z) * HD;
-                float2 * pml = (float2 *) (blk + (size_t) a.n_head * a.nsplit * HD) + (size_t) h * a.nsplit + blockIdx.z;
-                #pragma unroll
-                for (int dt = 0; dt < 8; dt++) po[16 * dt + i16] = o[u][dt][r];
-                if (i16 == 0) *pml = make_float2(mq, lq);
-            }
+    for (int r = 0; r < 4; r++) {
+        const float lq = __shfl(l_run, 4 * g + r), mq = __shfl(m_run, 4 * g + r);
+        const int row = rw + 4 * g + r;
+        if (row >= nrow) continue;
+        const int b = row / rep, h = kh * rep + (row - b * rep);
+        if (one) {
+            float * out = a.out + (size_t) b * a.n_head * HD + (size_t) h * HD;
+            #pragma unroll
+            for (int dt = 0; dt < 8; dt++) out[16 * dt + i16] = o[dt][r] / lq;
+        } else {
+            float * blk = a.part + (size_t) b * a.n_head * a.nsplit * (HD + 2);
+            float * po = blk + ((size_t) h * a.nsplit + blockIdx.z) * HD;
+            float2 * pml = (float2 *) (blk + (size_t) a.n_head * a.nsplit * HD) + (size_t) h * a.nsplit + blockIdx.z;
+            #pragma unroll
+            for (int dt = 0; dt < 8; dt++) po[16 * dt + i16] = o[dt][r];
+            if (i16 == 0) *pml = make_float2(mq, lq);
         }
     }
 }
