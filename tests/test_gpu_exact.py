@@ -423,14 +423,15 @@ def test_exact_greedy_64_equals_reference(decoder_file, name):
 
 @needs_ref
 @pytest.mark.parametrize("name,n", [("dense", 130), ("inorder", 64), ("qwenish", 77), ("dense_q8", 100)])
-def test_exact_batched_prompt_equals_reference(decoder_file, name, n):
-    """Exact mode reads a prompt batched (level 1: 64-position chunks through
-    the reference-order Q4 or Q8 GEMM, sml_xgemm_q4 / _q8, and the row form
-    of the reference-order attention), and its logits equal the reference
-    stepping the same ids through sml_forward bit for bit; so do 4 greedy
-    steps after it. Chunk boundaries inside the prompt (130 = 64 + 64 + 2),
+def test_exact_batched_prompt_equals_reference(decoder_file, monkeypatch, name, n):
+    """Exact mode reads a prompt batched (level 1: chunks, here of 64
+    positions, through the reference-order Q4 or Q8 GEMM, sml_pp_xgemm_q4 /
+    _q8, and the row form of the reference-order attention), and its logits
+    equal the reference stepping the same ids through sml_forward bit for bit;
+    so do 4 greedy steps after it. Chunk boundaries inside the prompt (130 = 64 + 64 + 2),
     one whole chunk (64), Qwen-shaped layers (77), Q8 layers (100). The same
     prompt read a token at a time (level 0) gives the same bits."""
+    monkeypatch.setenv("SML_PB", "64")
     p = decoder_file(name)
     V = DECODERS[name]["n_vocab"]
     ids = np.random.default_rng(n).integers(0, V, n).astype(np.int32)

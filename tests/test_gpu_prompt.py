@@ -1,4 +1,4 @@
-"""Prompt reading at level 2 on the GPU: the prompt MFMA GEMM (sml_pgemm_q4/_q6,
+"""Prompt reading at level 2 on the GPU: the prompt MFMA GEMM (sml_pp_sgemm_*,
 hundreds of positions per weight read) against the reference's own CPU
 kernels, and whole prompts against the reference's sml_prefill.
 
@@ -51,9 +51,9 @@ def ref_batch_sb(t, Q, S, U):
 @pytest.mark.parametrize("rows,cols,npos", [(1024, 4096, 512), (1000, 1536, 100), (4096, 14336, 77),
                                             (384, 8960, 17), (130, 256, 65)])
 def test_prompt_gemm_matches_reference(tmpdir_s, rows, cols, npos):
-    """sml_pgemm_q4 (through sml_hip_gemm_sb above 16 positions) against the
+    """sml_pp_sgemm_q4 (through sml_hip_gemm_sb above 16 positions) against the
     reference's flat4_sb kernel on the same per-256 activations, with ragged
-    row and position tiles (rows not a multiple of 128, positions not of 64)."""
+    row and position tiles (rows not a multiple of 64, positions not of 32)."""
     p = tmpdir_s / f"pg_{rows}_{cols}.ssf"
     if not p.exists():
         sa.synth_matrix(p, rows, cols, nbits=4, random_perm=False, seed=700 + cols + rows)
@@ -101,7 +101,7 @@ def test_prompt_gemm_swiglu_matches_reference(tmpdir_s, rows, cols, npos):
 @need_ref
 @pytest.mark.parametrize("rows,cols,npos", [(1024, 4096, 200), (1000, 1536, 100), (4096, 14336, 77), (130, 256, 65)])
 def test_prompt_gemm_q6_matches_reference(tmpdir_s, rows, cols, npos):
-    """sml_pgemm_q6 (6-bit codes: the 4-bit plane's nibble | the 2-bit plane's
+    """sml_pp_sgemm_q6 (6-bit codes: the 4-bit plane's nibble | the 2-bit plane's
     bits << 4, on the Q4 tile's integer superblock sums) against the
     reference's sml_matvec_batch_flat6_sb on the same per-256 activations,
     which sums the two planes' parts in separate fp32 passes: rel-RMS within
@@ -192,7 +192,7 @@ def test_level2_prompt_graded_against_reference(request, tmp_path_factory, model
     reference's sml_prefill in its default prompt regime: the logits after
     the prompt, then 8 steps on the reference's greedy ids, each graded
     (tiny_q6: the tiny model with 6-bit matrices).
-    The attention (a wave per position) and the fp32 sums run in their own
+    The attention (the MFMA flash kernel) and the fp32 sums run in their own
     orders, so an int8 activation code flips now and then; measured: prompt
     logits correlate at 0.99996 (tiny) and 0.99983 (Qwen-shaped layers), and
     one step in 27 picks another top-1 0.017 s.d. from the reference's (just
@@ -204,7 +204,7 @@ def test_level2_prompt_graded_against_reference(request, tmp_path_factory, model
     V = 2000 if model.startswith("tiny") else 32000
     path = d / f"{model}.ssf"
     if model.startswith("tiny"):
-        # tiny_q6: every matrix 6-bit (the prompt products on sml_pgemm_q6)
+        # tiny_q6: every matrix 6-bit (the prompt products on sml_pp_sgemm_q6)
         sa.synth_model(path, n_layer=2, n_embd=512, n_head=4, n_head_kv=2, n_ff=1024, n_vocab=V,
                        qkv_bias=True, random_perm=True, seed=31, nbits=6 if model == "tiny_q6" else 4)
     else:
@@ -284,7 +284,7 @@ def test_prompt_attention_4096(heads, n_rows, hd, flash, monkeypatch):
     """The level-2 prompt's causal attention on its own, at the end of a
     4096-position context: a chunk of n_rows positions ending at 4095 over a
     cache of random fp16 rows. The flash kernel splits the KV range as the
-    grid needs (32/8 heads: 2 splits at 512 rows, 16 at 64; 12/2 heads: 8)
+    grid needs (32/8 heads: 4 splits at 512 rows, 16 at 64; 12/2 heads: 11)
     and merges; the wave-per-position form splits by 128. Every chunk row's
     rotated K and its V as stored equal the oracle's bit for bit; sampled
     rows' outputs are within 1e-3 of the oracle's reference-order attention

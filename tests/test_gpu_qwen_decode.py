@@ -13,7 +13,7 @@ prompt with sml_prefill under SML_PROMPT_SB=0 (equal to stepping, bit for
 bit), then decodes with sml_forward; per step it keeps the greedy id, a
 digest of the logits' bytes, the top 8 and the logits' spread.
 
-- exact mode: the GPU reads the prompt (batched, in 64-position chunks of the
+- exact mode: the GPU reads the prompt (batched, in chunks of the
   reference-order GEMM and attention) and greedy-decodes on its own argmax;
   every step's logits have the reference's digest (equal bit for bit), so the
   ids are identical at every step.
