@@ -220,10 +220,11 @@ def moe_model(tmp_path_factory):
     return p
 
 
+@pytest.mark.parametrize("pb", ["16", ""])                # chunks of 16 positions, and the default's one
 @pytest.mark.parametrize("model", ["tiny", "tiny_inorder", "qwenish", "moe_model", "hd64"])
-def test_batched_prompt_equals_stepping(model, request):
-    """Batched prompt reading (level 1, the default): chunks of 16 positions
-    through the small-M GEMM and the causal attention read a prompt exactly
+def test_batched_prompt_equals_stepping(model, pb, request, monkeypatch):
+    """Batched prompt reading (level 1, the default): chunks of positions
+    through the batched GEMMs and the causal attention read a prompt exactly
     as stepping it does -- the logits of the last id bit for bit, for a first
     part and for a continuation of that prefix (37 ids: ragged chunks), and
     the same greedy continuation. Level 2 reads in the reference's per-256
@@ -231,6 +232,7 @@ def test_batched_prompt_equals_stepping(model, request):
     test_gpu_prompt.py), so against per-32 stepping it agrees to that
     regime's quantization: correlation above 0.999 and the same top-1
     unless the stepped logits are tied."""
+    monkeypatch.setenv("SML_PB", pb)
     p = request.getfixturevalue(model)
     V = 32000 if model == "qwenish" else 2000
     ids = np.random.default_rng(17).integers(0, V, 37).astype(np.int32)
@@ -255,12 +257,14 @@ def test_batched_prompt_equals_stepping(model, request):
             assert int(np.argmax(outs[2][i])) == int(np.argmax(ref)), f"level 2, part {i}"
 
 
+@pytest.mark.parametrize("pb", ["16", ""])
 @pytest.mark.parametrize("n", [16, 17, 33, 64])
-def test_batched_prompt_fills_context(tiny, n):
+def test_batched_prompt_fills_context(tiny, n, pb, monkeypatch):
     """Prompts that end exactly at n_ctx (the last position's K/V row is the
     cache's last), with whole and ragged chunks: level 1 equals stepping bit
     for bit, level 2 within its per-256 regime's quantization; a prompt past
     n_ctx is refused."""
+    monkeypatch.setenv("SML_PB", pb)
     ids = np.random.default_rng(n).integers(0, 2000, n).astype(np.int32)
     outs = {}
     for level in (0, 1, 2):
